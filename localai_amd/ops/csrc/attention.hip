@@ -11,12 +11,14 @@
 // * attn_decode: one query row per sequence.  Workgroup = (partition of <=PS keys, kv head,
 //   sequence); the G = Hq/Hkv query heads sharing a kv head are packed so K/V are read from
 //   HBM once (GQA packing).  Split-KV partials are merged by attn_decode_combine.
-// * attn_prefill: causal flash attention on MFMA (v_mfma_f32_16x16x32_bf16) for chunks of new
-//   tokens appended to a (possibly prefix-cached) context; K/V tiles of 32 keys come from the
-//   paged cache, so prefix reuse and chunked prefill need no special casing.
+// * attn_prefill: causal flash attention on MFMA for chunks of new tokens appended to a (possibly
+//   prefix-cached) context; K/V tiles come from the paged cache, so prefix reuse and chunked
+//   prefill need no special casing.  Plain softmax layers of width 64 and 128 run
+//   prefill_flash.h; score extras and other widths the 16x16x32 kernel below.
 #include <cstdlib>
 
 #include "common.h"
+#include "prefill_flash.h"
 
 namespace la {
 
@@ -857,6 +859,15 @@ extern "C" int la_attn_dense(const void* q, long ldq, const void* k, long ldk, c
   return (int)hipGetLastError();
 }
 
+// Query heads that share a workgroup's K and V in LDS (prefill_flash.h).  Four (eight waves, one workgroup per CU)
+// where a long context keeps every CU's loop busy; two workgroups of two per CU balance the shorter causal rows better
+// and hide each other's first loads (32 heads over 8: 2048 rows behind 10007 keys 455 us with 4, 492 with 2; one prompt
+// of 8000 622 / 653; 16 of 512 93 / 84; 64 of 128 60 / 51).  One for an odd number of heads per kv head.
+static int flash_heads(int ntiles, int Hq, int G, long keys) {
+  if (G % 4 == 0 && keys > 4096 && (long)ntiles * (Hq / 4) >= 256) return 4;
+  return G % 2 ? 1 : 2;
+}
+
 extern "C" int la_attn_prefill(const void* q, const void* kc, const void* vc, const int* tiles, int ntiles,
                                const int* cu_q, const int* ctx_lens, const int* block_tables, int max_blocks, int Hq,
                                int Hkv, int Dh, int BS, float scale, void* out, float softcap, int window,
@@ -865,6 +876,30 @@ extern "C" int la_attn_prefill(const void* q, const void* kc, const void* vc, co
   if (keep < 0 || Hq % Hkv || (dist_bias && nbias < 1) || (sink && sig) || chunk < 0 || (gate && ldg < (long)Hq * Dh)) return -1;
   const la::DecExtra E{dist_bias, nbias, sink, sig, chunk, (const bf16*)gate, ldg, keep};
   hipStream_t st = (hipStream_t)stream;
+  const int G = Hq / Hkv;
+  // plain causal softmax layers: prefill_flash.h.  Its K / V units are 16 keys of one page, hence the page sizes;
+  // softcaps, windows, gates and the other widths stay with the general kernel.
+  const bool plain = !dist_bias && !sink && !sig && !chunk && !gate && !keep && !(softcap > 0.f) && window <= 0;
+  if (plain && (Dh == 64 || Dh == 128) && scale > 0.f && BS >= 16 && !(BS & (BS - 1)) && ntiles <= 65535) {
+    const int hpw = flash_heads(ntiles, Hq, G, (long)max_blocks * BS);
+    const dim3 fg(Hq / hpw, ntiles);
+    const int shift = __builtin_ctz(BS);
+#define FL(D, H)                                                                                                  \
+  hipLaunchKernelGGL((la::prefill_flash_kernel<D, H>), fg, dim3(H * 128), 0, st, (const bf16*)q, (const bf16*)kc, \
+                     (const bf16*)vc, tiles, cu_q, ctx_lens, block_tables, max_blocks, Hq, Hkv, shift,            \
+                     scale * 1.4426950408889634f, (bf16*)out)
+#define FL_H(D)                \
+  do {                         \
+    if (hpw == 4) FL(D, 4);    \
+    else if (hpw == 2) FL(D, 2); \
+    else FL(D, 1);             \
+  } while (0)
+    if (Dh == 64) FL_H(64);
+    else FL_H(128);
+#undef FL_H
+#undef FL
+    return (int)hipGetLastError();
+  }
   dim3 grid(ntiles, Hq);
 #define PF_LAUNCH(D, SG)                                                                                          \
   hipLaunchKernelGGL((la::attn_prefill_kernel<D, false, SG>), grid, dim3(la::PF_T), 0, st, (const bf16*)q,        \
