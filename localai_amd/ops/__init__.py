@@ -66,6 +66,7 @@ def lib():
         P, I, F, LNG = ctypes.c_void_p, ctypes.c_int, ctypes.c_float, ctypes.c_long
         sig = {
             "la_qgemm_skinny": [I, P, P, P, P, I, I, P, I, I, I, P, I, LNG, P],
+            "la_qgemm_skinny_glu": [I, P, I, P, I, I, I, P, I, I, P, I, I, P],
             "la_qgemv_dp4": [I, P, P, P, I, P, I, I, I, P, I, LNG, P, LNG, I, P, I, P],
             "la_moe_gemv": [I, I, P, I, I, I, P, I, I, P, I, I, P, LNG, I, I, P, P, I, LNG, P],
             "la_gemv_variant": [I],
@@ -1051,6 +1052,11 @@ def _autotune_mid(x, ws, key, Ntot):
     return best
 
 
+def _skinny_ok(w: QWeight) -> bool:
+    """Can gemm_skinny.hip read w: whole super-blocks, and of Q6_K an even number (it reads pairs of their scales)."""
+    return w.K % 256 == 0 and not (w.fmt == FMT_Q6_K and w.N * (w.K // 256) % 2)
+
+
 def linear(x: torch.Tensor, w: QWeight, bias: Optional[torch.Tensor] = None,
            out_slabs: Optional[torch.Tensor] = None, force: Optional[str] = None) -> Partial:
     """y = x @ W^T.  x: [M, K] bf16.  GPU: M <= 2 -> int8-dot GEMV, M <= 64 -> skinny MFMA
@@ -1078,7 +1084,7 @@ def linear_multi(x: torch.Tensor, ws: Sequence[QWeight], bias: Optional[torch.Te
         raise ValueError("linear: x must be contiguous bf16")
     if any(w.fmt == FMT_F32 for w in ws):
         raise ValueError("linear: fp32 weights take fp32 activations")
-    skinny_ok = all(w.K % 256 == 0 for w in ws) and _has("la_qgemm_skinny")
+    skinny_ok = all(_skinny_ok(w) for w in ws) and _has("la_qgemm_skinny")
     use_skinny = (M <= SKINNY_MAX_M and skinny_ok) if force is None else force == "skinny"
     tile_ok = TILE_GEMM and all(w.tile_ok for w in ws) and (_has("la_qgemm_tile") or _has("la_qgemm32") or _has("la_bsgemm"))
     S, tile, kind = 0, 0, None
@@ -1181,6 +1187,16 @@ def _run_glu(x: torch.Tensor, pair, F: int, mode: int, tile: int, out: torch.Ten
                               mode, tile, _stream()), "la_qgemm_glu")
 
 
+def _run_skinny_glu(x: torch.Tensor, pair, F: int, mode: int, out: torch.Tensor) -> None:
+    M, K = x.shape
+    if x.dtype != torch.bfloat16 or not x.is_contiguous() or K != pair[0].K:
+        raise ValueError("glu_linear: x must be contiguous bf16 [M, K]")
+    wa, oa, wb, ob = pair
+    a, b = ((ctypes.c_void_p * 4)(*w.ptrs()) for w in (wa, wb))
+    _check(lib().la_qgemm_skinny_glu(wa.fmt, a, oa, b, ob, F, K, x.data_ptr(), K, M, out.data_ptr(), F, mode, _stream()),
+           "la_qgemm_skinny_glu")
+
+
 def _time_cold(fn) -> float:
     fn()
     ts = []
@@ -1198,19 +1214,27 @@ def _time_cold(fn) -> float:
 def glu_linear(x: torch.Tensor, ws: Sequence[QWeight], F: int, mode: int,
                bias: Optional[torch.Tensor] = None) -> Optional[torch.Tensor]:
     """act(x Wg^T) * (x Wu^T) -> bf16 [M, F] in ONE tile-GEMM launch with the GLU activation in
-    its epilogue (gate and up columns of the same index share a tile), for decode batches.  The
-    autotuner times it against the unfused pair (tuned GEMM + activation kernel) once per
-    32-row bucket; returns None where the fused kernel does not apply or loses."""
+    its epilogue (gate and up columns of the same index share a tile), for decode batches.  Up to
+    SKINNY_MAX_M rows gemm_skinny.hip's gated form, which is the faster one at every size (28672 x
+    4096, Q4_K: 23 us for up to 16 rows against 28 + 5 for product and activation, 33 against 43 +
+    5 at 50).  Above, the autotuner times it against the unfused pair (tuned GEMM + activation
+    kernel) once per 32-row bucket; returns None where the fused kernel does not apply or loses."""
     if not (GLU_FUSE and TILE_GEMM and x.is_cuda and bias is None and mode in GLU_ACTS):
         return None
     M, K = x.shape
-    if M > MID_MAX_M or M <= SKINNY_MAX_M:
+    if M > MID_MAX_M:
         # prefill chunks: dequant + hipBLASLt + the activation kernel beats every fused GLU tile
         # at M >= 1024 (gemm_bs.hip's GLU mode included, profiles/r6_gemm_bs.md)
         return None
     pair = _glu_pair(ws, F)
     if pair is None:
         return None
+    if M <= SKINNY_MAX_M:
+        if not _has("la_qgemm_skinny_glu") or not all(_skinny_ok(w) for w in ws) or (GEMV_DP4 and M <= GEMV_MAX_M and all(w.gemv_ok for w in ws)):
+            return None   # one or two rows: the int8-dot GEMVs, with the activation in the down projection's prologue
+        out = torch.empty(M, F, dtype=torch.bfloat16, device=x.device)
+        _run_skinny_glu(x, pair, F, mode, out)
+        return out
     key = ((M + 31) // 32 * 32, K, F, mode, tuple((w.fmt, w.N) for w in ws))
     if key not in _GLU_CHOICE:
         if not GEMM_AUTOTUNE or torch.cuda.is_current_stream_capturing():

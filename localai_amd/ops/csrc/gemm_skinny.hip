@@ -1,140 +1,423 @@
 // Quantised "skinny" GEMM for decode / small batches:  out[s][m][n] = sum_{k in split s} X[m,k] * W[n,k]
+// and its gated form                                   out[m][j]    = act(x Wg[j]^T) * (x Wu[j]^T)   (bf16)
 //
 // Replaces ggml-cuda's mmvq/mmq ([external]).  MI355X-first design:
-//  * B operand = weights, read ONCE from HBM straight into VGPRs (16-byte loads,
-//    one super-block of prefetch in flight), dequantised in-register to bf16 and fed
-//    to v_mfma_f32_16x16x32_bf16.  No LDS round trip for weights (guide §5:
-//    "GEMV / M <= 16 decode weights: load straight to VGPRs").
-//  * A operand = activations (M <= 64 rows), staged per super-block through LDS
-//    (shared by the 4 waves of the workgroup, each wave owns 16 output columns),
-//    issue-early / write-late (T14) so the L2 latency of X hides under the MFMAs.
-//  * Split-K over grid.y gives >= 2 workgroups per CU; partial fp32 slabs are summed by
-//    the consuming kernel (rmsnorm / rope / silu-mul prologue), never by atomics.
+//  * A workgroup of 4 waves owns 64 NW output columns (wave: NW tiles of 16) and all M <= 64 rows; a stage is 128 k.
+//  * Weights and activations arrive by LDS-DMA in NS-slot rings.  A weight row's bytes of a stage are contiguous (64
+//    of Q4_K), so an instruction reads whole 64-byte pieces of 16 rows: with each lane loading its own fragment
+//    straight to registers neighbouring lanes are in different rows, every lane is a line look-up of its own, and
+//    that, not HBM, was the bound (390 cycles of the CU's address path per 16 x 256 weights; about 110 here).
+//  * A wave dequantises its own columns to bf16 for v_mfma_f32_16x16x32_bf16; the raw bytes are private to the wave,
+//    the activations shared by the 4 waves; counted vmcnt, one barrier per stage.
+//  * 16-byte chunks are exchanged inside their row by an XOR on the SOURCE address, chosen so that the lanes which
+//    ds_read_b128 serves together (0-3, 12-15, 20-27; 4-11, 16-19, 28-31; the same + 32) hit different banks.
+//  * A stage's weights are read from LDS an iteration before they are used, and all its activations before the first
+//    product, so the vector pipe does not wait for LDS between its dequantisations.
+//  * K is split over grid.y where the columns leave CUs idle: fp32 slabs summed by the consuming kernel (rmsnorm /
+//    rope prologue), never by atomics.
+// What bounds it: 28672 x 4096 of Q4_K (74 MB) gated, 4 to 16 rows: 23.4 us, of which 16.5 remain without the
+// arithmetic (2.6 vector instructions a weight: about 10 us of every SIMD).  Before: 28.5 us ungated and 4.6 for the
+// activation kernel; 50 rows 43 + 4.8 -> 33; 128256 x 4096 of Q6_K, 16 rows: 131 -> 113; 4096 x 14336 of Q6_K:
+// 22.4 -> 17.5; the gated 8-bit form 38 + 4.6 -> 27.5.
 #include "qweight.h"
 
 namespace la {
 
-constexpr int SK_WAVES = 4;
-constexpr int SK_THREADS = 64 * SK_WAVES;
-constexpr int SK_LDS_STRIDE = 256 + 8;  // bf16 elements per LDS row (16 B pad: spreads banks)
+constexpr int SK_K = 128;              // k of one stage
 
-template <int FMT, int MT>
-__global__ __launch_bounds__(SK_THREADS, 2) void qgemm_skinny_kernel(
-    QW w, const bf16* __restrict__ X, int ldx, int M, int k_per_split, float* __restrict__ out, int ldo,
-    long slab) {
-  constexpr int MP = 16 * MT;
-  __shared__ __attribute__((aligned(16))) bf16 xs[MP * SK_LDS_STRIDE];
+LA_DEV void sk_dma16(const void* g, void* l) {
+  __builtin_amdgcn_global_load_lds(g, (__attribute__((address_space(3))) void*)l, 16, 0, 0);
+}
+LA_DEV void sk_dma4(const void* g, void* l) {
+  __builtin_amdgcn_global_load_lds(g, (__attribute__((address_space(3))) void*)l, 4, 0, 0);
+}
 
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int g = lane >> 4, r = lane & 15;
-  const int N = w.N, K = w.K;
-  const int split = blockIdx.y;
-  const int kbeg = split * k_per_split;
-  const int nsb = min(k_per_split, K - kbeg) >> 8;
-  const int n = blockIdx.x * (16 * SK_WAVES) + wave * 16 + r;
-  const int nl = min(n, N - 1);  // clamp: out-of-range lanes compute garbage, never stored
+// Rows 0-3, 12-15 and 4-11 each numbered 0 .. 7: the two sets of rows that one phase reads at chunks c and c ^ d.
+// sk_rot spreads them over the 8 chunks of which bit d is clear.
+LA_DEV int sk_idx(int r) { return (r & 3) | ((r & 8) >> 1); }
+template <int D>
+LA_DEV int sk_rot(int r) {
+  const int i = sk_idx(r);
+  return D == 1 ? i << 1 : D == 2 ? (i & 1) | ((i & 6) << 1) : (i & 3) | ((i & 4) << 1);
+}
 
-  // ---- X staging: MP rows x 256 cols bf16 = MP*32 16-byte chunks per super-block
-  constexpr int XCH = MP * 32;
-  constexpr int XPT = (XCH + SK_THREADS - 1) / SK_THREADS;
-  bf16x8 xr[XPT];
-  auto x_issue = [&](int sb) {
-#pragma unroll
-    for (int i = 0; i < XPT; ++i) {
-      const int c = tid + i * SK_THREADS;
-      const int row = c >> 5, col = (c & 31) * 8;
-      bf16x8 v = {};
-      if (c < XCH && row < M) v = *(const bf16x8*)(X + (size_t)row * ldx + kbeg + sb * 256 + col);
-      xr[i] = v;
-    }
+// Per format: the 16 weight rows of a tile over one stage.  ptr(): this lane's source addresses (row(i): row i of the
+// tile); issue(): DMA of stage ks to dst; issue_quad(): of the scales of four super-blocks; load() / prep() / deq<S>(): lane (g, r)'s 32 weights of row r,
+// 8 for each of the 4 MFMA steps; chunk(s, g): which 8 k of the stage those are.
+template <int FMT> struct SkW;
+
+// Scales are fetched for four super-blocks (a quad: 8 stages) at a time, 64 bytes of a row's scale plane: by the stage
+// every row would cost two more requests of 4 or 8 bytes, three times as many in all.  Row r's 16 bytes of super-block i
+// of the quad lie at 64 r + 16 (i ^ (r >> 2)).
+LA_DEV int sk_quad(int r, int i) { return 64 * r + 16 * (i ^ (r >> 2)); }
+
+// Q4_K: 64 bytes a row (two groups of 32: low nibbles the first 32 k, high nibbles the next), 4 (sc, m) pairs, d, dmin.
+// Lane g: bytes 16 g .. 16 g + 15, i.e. 16 k of the blocks 2 (g >> 1) and 2 (g >> 1) + 1.  Codes 0 .. 15 read as fp8
+// e4m3 are exactly code / 512, so one v_cvt_pk_f32_fp8 makes two of them.
+template <> struct SkW<FMT_Q4_K> {
+  static constexpr int BYTES = 1024, PIECES = 1, XD = 2, QBYTES = 1024 + 256;
+  LA_DEV static int chunk(int s, int g) { return 8 * (g >> 1) + 4 * (s >> 1) + 2 * (g & 1) + (s & 1); }
+  struct Ptr {
+    const uint8_t *raw, *scm, *dd;
+    int nsb, qi;
   };
-  auto x_store = [&]() {
+  template <typename Row>
+  LA_DEV static Ptr ptr(const QW& w, int lane, Row row) {
+    Ptr p;
+    const int rr = lane >> 2;
+    p.nsb = w.K >> 8;
+    p.qi = (lane & 3) ^ (rr >> 2);
+    p.raw = w.p0 + (size_t)row(rr) * (w.K >> 1) + 16 * ((lane & 3) ^ (2 * (rr >> 3)));
+    p.scm = w.p2 + (size_t)row(rr) * p.nsb * 16;
+    p.dd = w.p3 + (size_t)row(rr) * p.nsb * 4;
+    return p;
+  }
+  LA_DEV static void issue(const Ptr& p, int ks, uint8_t* dst) { sk_dma16(p.raw + 64 * ks, dst); }
+  LA_DEV static void issue_quad(const Ptr& p, int sb, uint8_t* dst, int lane) {
+    sk_dma16(p.scm + 16 * min(sb + p.qi, p.nsb - 1), dst);
+    sk_dma4(p.dd + 4 * min(sb + (lane & 3), p.nsb - 1), dst + 1024);
+  }
+  u32x4 q;
+  uint32_t scm, dd;
+  float D[2], Mn[2];
+  LA_DEV void load(const uint8_t* l, const uint8_t* qd, int t, int r, int g, int, int) {
+    const int i = (t >> 1) & 3;
+    q = *(const u32x4*)(l + 64 * r + 16 * (g ^ (2 * (r >> 3))));
+    scm = *(const uint32_t*)(qd + sk_quad(r, i) + 8 * (t & 1) + 4 * (g >> 1));
+    dd = *(const uint32_t*)(qd + 1024 + 16 * r + 4 * i);
+  }
+  LA_DEV void prep(int) {
+    const float d = h2f(dd & 0xFFFFu) * 512.f, dmin = -h2f(dd >> 16);
+    D[0] = d * ubyte_f(scm, 0);
+    Mn[0] = dmin * ubyte_f(scm, 1);
+    D[1] = d * ubyte_f(scm, 2);
+    Mn[1] = dmin * ubyte_f(scm, 3);
+  }
+  template <int S>
+  LA_DEV bf16x8 deq() const {
+    typedef float f32x2 __attribute__((ext_vector_type(2)));
+    constexpr int h = S >> 1;
+    const uint32_t a = ((S & 1 ? q.z : q.x) >> (4 * h)) & 0x0F0F0F0Fu, b = ((S & 1 ? q.w : q.y) >> (4 * h)) & 0x0F0F0F0Fu;
+    const f32x2 a0 = __builtin_amdgcn_cvt_pk_f32_fp8(a, false), a1 = __builtin_amdgcn_cvt_pk_f32_fp8(a, true);
+    const f32x2 b0 = __builtin_amdgcn_cvt_pk_f32_fp8(b, false), b1 = __builtin_amdgcn_cvt_pk_f32_fp8(b, true);
+    const u32x4 v = {pk_bf16(fmaf(D[h], a0.x, Mn[h]), fmaf(D[h], a0.y, Mn[h])),
+                     pk_bf16(fmaf(D[h], a1.x, Mn[h]), fmaf(D[h], a1.y, Mn[h])),
+                     pk_bf16(fmaf(D[h], b0.x, Mn[h]), fmaf(D[h], b0.y, Mn[h])),
+                     pk_bf16(fmaf(D[h], b1.x, Mn[h]), fmaf(D[h], b1.y, Mn[h]))};
+    return __builtin_bit_cast(bf16x8, v);
+  }
+};
+
+// Q6_K: a stage is one 128-half of the block: ql 64 bytes (l and 32 + l; low nibbles k 0-63, high 64-127), qh 32 bytes
+// (2 bits for each quarter of 32 k), 8 scales of 16 k, d.  Lane g: l = 8 g .. 8 g + 7, step s the quarter s.
+template <> struct SkW<FMT_Q6_K> {
+  static constexpr int BYTES = 1024 + 512, PIECES = 2, XD = 1, QBYTES = 1024 + 256;
+  LA_DEV static int chunk(int s, int g) { return 4 * s + g; }
+  struct Ptr {
+    const uint8_t *ql, *qh, *sc, *d;
+    int nsb, qi, idx, last;   // idx: the row's first index in the plane of 2-byte scales, last: the plane's last dword
+  };
+  template <typename Row>
+  LA_DEV static Ptr ptr(const QW& w, int lane, Row row) {
+    Ptr p;
+    const int rr = lane >> 2, rh = (lane & 31) >> 1;
+    p.nsb = w.K >> 8;
+    p.qi = (lane & 3) ^ (rr >> 2);
+    p.ql = w.p0 + (size_t)row(rr) * (w.K >> 1) + 16 * ((lane & 3) ^ (rr >> 2));
+    p.qh = w.p1 + (size_t)row(rh) * (w.K >> 2) + 16 * ((lane & 1) ^ (rh >> 3));
+    p.sc = w.p2 + (size_t)row(rr) * p.nsb * 16;
+    p.d = w.p3;
+    p.idx = row(rr) * p.nsb;
+    p.last = (w.N * p.nsb >> 1) - 1;
+    return p;
+  }
+  LA_DEV static void issue(const Ptr& p, int ks, uint8_t* dst) {
+    sk_dma16(p.ql + 64 * ks, dst);
+    if ((threadIdx.x & 63) < 32) sk_dma16(p.qh + 32 * ks, dst + 1024);
+  }
+  // d is 2 bytes at any even address: the aligned dwords that hold a row's four of them (three at most)
+  LA_DEV static void issue_quad(const Ptr& p, int sb, uint8_t* dst, int lane) {
+    sk_dma16(p.sc + 16 * min(sb + p.qi, p.nsb - 1), dst);
+    sk_dma4(p.d + 4 * (size_t)min(((p.idx + sb) >> 1) + (lane & 3), p.last), dst + 1024);
+  }
+  u32x2 la, lb, qh, sc;
+  uint16_t dbits;
+  float S[4];
+  LA_DEV void load(const uint8_t* l, const uint8_t* qd, int t, int r, int g, int idx, int sb) {
+    const int i = (t >> 1) & 3;
+    const uint8_t* b = l + 64 * r + 8 * (g & 1);
+    la = *(const u32x2*)(b + 16 * ((g >> 1) ^ (r >> 2)));
+    lb = *(const u32x2*)(b + 16 * ((2 + (g >> 1)) ^ (r >> 2)));
+    qh = *(const u32x2*)(l + 1024 + 32 * r + 16 * ((g >> 1) ^ (r >> 3)) + 8 * (g & 1));
+    sc = *(const u32x2*)(qd + sk_quad(r, i) + 8 * (t & 1));
+    const int q0 = idx + sb - i, e = idx + sb;     // the quad's first and this super-block's place in the plane
+    dbits = *(const uint16_t*)(qd + 1024 + 16 * r + 4 * ((e >> 1) - (q0 >> 1)) + 2 * (e & 1));
+  }
+  LA_DEV void prep(int g) {
+    const float d = h2f(dbits);
+    const int sh = 8 * (g >> 1);
+    S[0] = d * (float)((int)(sc.x << (24 - sh)) >> 24);
+    S[1] = d * (float)((int)(sc.x << (8 - sh)) >> 24);
+    S[2] = d * (float)((int)(sc.y << (24 - sh)) >> 24);
+    S[3] = d * (float)((int)(sc.y << (8 - sh)) >> 24);
+  }
+  template <int St>
+  LA_DEV bf16x8 deq() const {
+    const u32x2 L = (St & 1) ? lb : la;
+    constexpr int ls = 4 * (St >> 1), hs = 2 * St;
+    const uint32_t u0 = opaque(((L.x >> ls) & 0x0F0F0F0Fu) | (((qh.x >> hs) & 0x03030303u) << 4));
+    const uint32_t u1 = opaque(((L.y >> ls) & 0x0F0F0F0Fu) | (((qh.y >> hs) & 0x03030303u) << 4));
+    return bytes_bf16(u0, u1, S[St], -32.f * S[St]);
+  }
+};
+
+// Q8_0: 128 bytes and 4 scales a row.  Lane g: block g.
+template <> struct SkW<FMT_Q8_0> {
+  static constexpr int BYTES = 2048, PIECES = 2, XD = 4, QBYTES = 1024;
+  LA_DEV static int chunk(int s, int g) { return 4 * g + s; }
+  // 8 chunks a row, 2 g and 2 g + 1 read: as sk_rot with 3 bits, bit 1 clear, for the 8 rows of one parity
+  LA_DEV static int rot(int r) { return ((r >> 1) & 1) | (((r >> 3) & 1) << 2); }
+  struct Ptr {
+    const uint8_t *a, *b, *d;
+    int nsb, qi;
+  };
+  template <typename Row>
+  LA_DEV static Ptr ptr(const QW& w, int lane, Row row) {
+    Ptr p;
+    const int rr = lane >> 3;
+    p.nsb = w.K >> 8;
+    p.qi = (lane & 3) ^ (lane >> 4);
+    p.a = w.p0 + (size_t)row(rr) * w.K + 16 * ((lane & 7) ^ rot(rr));
+    p.b = w.p0 + (size_t)row(8 + rr) * w.K + 16 * ((lane & 7) ^ rot(8 + rr));
+    p.d = w.p1 + (size_t)row(lane >> 2) * p.nsb * 16;
+    return p;
+  }
+  LA_DEV static void issue(const Ptr& p, int ks, uint8_t* dst) {
+    sk_dma16(p.a + 128 * ks, dst);
+    sk_dma16(p.b + 128 * ks, dst + 1024);
+  }
+  LA_DEV static void issue_quad(const Ptr& p, int sb, uint8_t* dst, int) {
+    sk_dma16(p.d + 16 * min(sb + p.qi, p.nsb - 1), dst);
+  }
+  u32x4 a, b;
+  uint16_t dbits;
+  float d;
+  LA_DEV void load(const uint8_t* l, const uint8_t* qd, int t, int r, int g, int, int) {
+    a = *(const u32x4*)(l + 128 * r + 16 * ((2 * g) ^ rot(r)));
+    b = *(const u32x4*)(l + 128 * r + 16 * ((2 * g + 1) ^ rot(r)));
+    dbits = *(const uint16_t*)(qd + sk_quad(r, (t >> 1) & 3) + 8 * (t & 1) + 2 * g);
+  }
+  LA_DEV void prep(int) {
+    d = h2f(dbits);
+  }
+  template <int S>
+  LA_DEV bf16x8 deq() const {
+    const u32x4 v = S < 2 ? a : b;
+    const uint32_t lo = (S & 1) ? v.z : v.x, hi = (S & 1) ? v.w : v.y;
+    // signed bytes with the sign bit flipped: 0 .. 255, 128 too much
+    return bytes_bf16(opaque(lo ^ 0x80808080u), opaque(hi ^ 0x80808080u), d, -128.f * d);
+  }
+};
+
+template <> struct SkW<FMT_BF16> {
+  static constexpr int BYTES = 4096, PIECES = 4, XD = 4, QBYTES = 0;
+  LA_DEV static int chunk(int s, int g) { return 4 * g + s; }
+  struct Ptr {
+    const uint8_t* p[4];
+  };
+  template <typename Row>
+  LA_DEV static Ptr ptr(const QW& w, int lane, Row row) {
+    Ptr p;
 #pragma unroll
-    for (int i = 0; i < XPT; ++i) {
-      const int c = tid + i * SK_THREADS;
-      if (c < XCH) {
-        const int row = c >> 5, col = (c & 31) * 8;
-        *(bf16x8*)(xs + row * SK_LDS_STRIDE + col) = xr[i];
-      }
+    for (int i = 0; i < 4; ++i) {
+      const int rr = 4 * i + (lane >> 4);
+      p.p[i] = w.p0 + (size_t)row(rr) * w.K * 2 + 16 * ((lane & 15) ^ sk_rot<XD>(rr));
     }
+    return p;
+  }
+  LA_DEV static void issue(const Ptr& p, int ks, uint8_t* dst) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) sk_dma16(p.p[i] + 256 * ks, dst + 1024 * i);
+  }
+  LA_DEV static void issue_quad(const Ptr&, int, uint8_t*, int) {}
+  bf16x8 v[4];
+  LA_DEV void prep(int) {}
+  LA_DEV void load(const uint8_t* l, const uint8_t*, int, int r, int g, int, int) {
+#pragma unroll
+    for (int s = 0; s < 4; ++s) v[s] = *(const bf16x8*)(l + 256 * r + 16 * (chunk(s, g) ^ sk_rot<XD>(r)));
+  }
+  template <int S>
+  LA_DEV bf16x8 deq() const { return v[S]; }
+};
+
+// The gated form's second weight: gate rows oa .. oa + F of the first, up rows ob .. ob + F of this one.
+struct SkGlu {
+  QW b;
+  int oa, ob, F, act;
+  bf16* out;
+};
+
+LA_DEV float sk_gelu_tanh(float x) { return 0.5f * x * (1.f + tanhf(0.7978845608f * (x + 0.044715f * x * x * x))); }
+
+template <int FMT, int MT, int WV, bool GLU>
+struct SkCfg {
+  using W = SkW<FMT>;
+  static constexpr int XB = 16 * MT * SK_K * 2, SLOT = XB + WV * W::BYTES, QUADS = 2 * WV * W::QBYTES;
+  // slots of the ring: for two to three workgroups of 4 waves a CU, or one of 8
+  static constexpr int WANT = ((WV == 8 ? 150 : 52) * 1024 - QUADS) / SLOT;
+  static constexpr int FIT = (160 * 1024 - QUADS) / SLOT;
+  static constexpr int NS = WANT >= 4 ? (WANT > 8 ? 8 : WANT) : FIT < 4 ? FIT : 4;
+  static_assert(NS >= 3, "ring");
+};
+
+template <int FMT, int MT, int WV, bool GLU>
+__global__ __launch_bounds__(64 * WV, 2) void qgemm_skinny_kernel(
+    QW w, const bf16* __restrict__ X, int ldx, int M, int k_per_split, float* __restrict__ out, int ldo,
+    long slab, SkGlu glu) {
+  static_assert(!GLU || WV == 8, "4 waves of gate and 4 of up tiles");
+  using W = SkW<FMT>;
+  using C = SkCfg<FMT, MT, WV, GLU>;
+  constexpr int NS = C::NS;
+  constexpr int PX = 4 * MT < WV ? 1 : 4 * MT / WV;    // pieces (4 rows) of X a wave fetches; MT 1, 8 waves: each by two
+  constexpr int L = PX + W::PIECES;                    // DMAs of a wave per stage
+  static_assert((NS - 3) * L < 64 && NS <= 8, "vmcnt; a quad's scales have landed 8 stages later");
+  __shared__ __attribute__((aligned(1024))) uint8_t lds[NS * C::SLOT + C::QUADS];
+
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int g = lane >> 4, r = lane & 15;
+  const int N = GLU ? glu.F : w.N;
+  const int nst = k_per_split / SK_K, ks0 = blockIdx.y * nst;
+  const bool up = GLU && wave >= 4;
+  const int c0 = GLU ? (blockIdx.x * 4 + (wave & 3)) * 16 : (blockIdx.x * WV + wave) * 16;   // the wave's first column
+
+  // sources: pieces of X, the tile's planes (rows past N repeat the last)
+  const bf16* xp[PX];
+#pragma unroll
+  for (int i = 0; i < PX; ++i) {
+    const int row = 4 * ((wave * PX + i) % (4 * MT)) + (lane >> 4);
+    xp[i] = X + (size_t)min(row, M - 1) * ldx + ((lane & 15) ^ sk_rot<W::XD>(row & 15)) * 8;
+  }
+  const QW wt = up ? glu.b : w;
+  auto row = [&](int i) { return (GLU ? (up ? glu.ob : glu.oa) : 0) + min(c0 + i, N - 1); };
+  const typename W::Ptr wp = W::ptr(wt, lane, row);
+  const int idx = row(r) * (w.K >> 8);
+  auto issue = [&](int t, int slot) {        // (clamped, never behind a branch: the count of DMAs in flight is fixed)
+    uint8_t* s = lds + slot * C::SLOT;
+    const int ks = ks0 + min(t, nst - 1);
+#pragma unroll
+    for (int i = 0; i < PX; ++i) sk_dma16(xp[i] + ks * SK_K, s + ((wave * PX + i) % (4 * MT)) * 1024);
+    W::issue(wp, ks, s + C::XB + wave * W::BYTES);
+  };
+  uint8_t* quads = lds + NS * C::SLOT + wave * (2 * W::QBYTES);
+  auto issue_quad = [&](int t, int buf) {    // scales of the stages t .. t + 7
+    W::issue_quad(wp, (ks0 + t) >> 1, quads + buf * W::QBYTES, lane);
+  };
+  auto fetch = [&](W& f, int t, int slot) {
+    f.load(lds + slot * C::SLOT + C::XB + wave * W::BYTES, quads + ((t >> 3) & 1) * W::QBYTES, t, r, g, idx, (ks0 + t) >> 1);
   };
 
   f32x4 acc[MT];
 #pragma unroll
   for (int i = 0; i < MT; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+  int xoff[4];
+#pragma unroll
+  for (int s = 0; s < 4; ++s) xoff[s] = r * (SK_K * 2) + 16 * (W::chunk(s, g) ^ sk_rot<W::XD>(r));
 
-  const int sb0 = kbeg >> 8;
-  WFrag<FMT> fa, fb;
-  x_issue(0);
-  fa.load(w, nl, sb0, g);
-
-  auto compute = [&](WFrag<FMT>& f) {
-    f.prep(g);
-#define SK_STEP(S)                                                                         \
-  {                                                                                        \
-    const bf16x8 b = f.template deq<S>();                                                  \
-    const int kp = kphys<FMT>(S, g);                                                       \
-    _Pragma("unroll") for (int mt = 0; mt < MT; ++mt) {                                    \
-      const bf16x8 a = *(const bf16x8*)(xs + (mt * 16 + r) * SK_LDS_STRIDE + kp);          \
-      acc[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc[mt], 0, 0, 0);           \
-    }                                                                                      \
+  issue_quad(0, 0);
+#pragma unroll
+  for (int t = 0; t < NS - 1; ++t) issue(t, t);
+  W f[2];
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NS - 2) * L) : "memory");
+  fetch(f[0], 0, 0);
+  int slot = 0;
+  // Iteration t multiplies stage t: its weights are in registers, read from LDS during iteration t - 1
+  auto step = [&](W& cur, W& nxt, int t) {
+    // this wave's part of stage t + 1 has landed; with the barrier everyone's part of stage t has (waited for an
+    // iteration ago), and the slot of stage t - 1 is free
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((NS - 3) * L) : "memory");
+    if ((t & 7) == 0) issue_quad(t + 8, ((t >> 3) + 1) & 1);
+    issue(t + NS - 1, slot == 0 ? NS - 1 : slot - 1);
+    const uint8_t* s = lds + slot * C::SLOT;
+    bf16x8 a[4][MT];
+    slot = slot == NS - 1 ? 0 : slot + 1;
+#pragma unroll
+    for (int q = 0; q < (MT > 2 ? 1 : 4); ++q)
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt) a[q][mt] = *(const bf16x8*)(s + xoff[q] + mt * (16 * SK_K * 2));
+    fetch(nxt, t + 1, slot);
+    __builtin_amdgcn_sched_barrier(0);
+    cur.prep(g);
+#define SK_STEP(S)                                                                                    \
+  {                                                                                                   \
+    if constexpr (MT > 2 && S < 3) {                                                                  \
+      _Pragma("unroll") for (int mt = 0; mt < MT; ++mt)                                               \
+        a[S + 1][mt] = *(const bf16x8*)(s + xoff[S + 1] + mt * (16 * SK_K * 2));                      \
+    }                                                                                                 \
+    const bf16x8 b = cur.template deq<S>();                                                           \
+    _Pragma("unroll") for (int mt = 0; mt < MT; ++mt)                                                 \
+      acc[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[S][mt], b, acc[mt], 0, 0, 0);               \
   }
-    SK_STEP(0) SK_STEP(1) SK_STEP(2) SK_STEP(3) SK_STEP(4) SK_STEP(5) SK_STEP(6) SK_STEP(7)
+    SK_STEP(0) SK_STEP(1) SK_STEP(2) SK_STEP(3)
 #undef SK_STEP
   };
-
-  // two super-blocks per iteration with statically named fragments (no runtime-indexed arrays)
-  for (int sb = 0; sb < nsb; sb += 2) {
-    // --- super-block sb (fragment fa)
-    __syncthreads();  // previous readers of xs done
-    x_store();
-    __syncthreads();
-    if (sb + 1 < nsb) {
-      x_issue(sb + 1);
-      fb.load(w, nl, sb0 + sb + 1, g);
-    }
-    compute(fa);
-    if (sb + 1 >= nsb) break;
-    // --- super-block sb+1 (fragment fb)
-    __syncthreads();
-    x_store();
-    __syncthreads();
-    if (sb + 2 < nsb) {
-      x_issue(sb + 2);
-      fa.load(w, nl, sb0 + sb + 2, g);
-    }
-    compute(fb);
+  for (int t = 0; t < nst; t += 2) {         // (a split is whole super-blocks: an even number of stages)
+    step(f[0], f[1], t);
+    step(f[1], f[0], t + 1);
   }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the clamped last stages: nothing may land after the wave's end
 
-  if (n < N) {
-    float* o = out + (size_t)split * slab;
+  const int n = c0 + r;
+  if constexpr (GLU) {
+    __syncthreads();
+    f32x4* ex = (f32x4*)lds;
+    if (up) {
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt) ex[((wave - 4) * MT + mt) * 64 + lane] = acc[mt];
+    }
+    __syncthreads();
+    if (up || n >= N) return;
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) {
+      const f32x4 u = ex[(wave * MT + mt) * 64 + lane];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int m = mt * 16 + 4 * g + i;
+        const float a = glu.act == 0 ? silu(acc[mt][i]) : sk_gelu_tanh(acc[mt][i]);
+        if (m < M) glu.out[(size_t)m * ldo + n] = (bf16)(a * u[i]);
+      }
+    }
+  } else {
+    if (n >= N) return;
+    float* o = out + (size_t)blockIdx.y * slab;
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const int m = mt * 16 + 4 * g + i;
         if (m < M) o[(size_t)m * ldo + n] = acc[mt][i];
       }
-    }
   }
 }
 
-template <int FMT, int MT>
-static void launch_skinny_t(const QW& w, const bf16* X, int ldx, int M, int splits, float* out, int ldo,
-                            long slab, hipStream_t st) {
-  const int nsb_total = w.K >> 8;
-  const int per = nsb_total / splits;
-  dim3 grid((w.N + 16 * SK_WAVES - 1) / (16 * SK_WAVES), splits);
-  hipLaunchKernelGGL((qgemm_skinny_kernel<FMT, MT>), grid, dim3(SK_THREADS), 0, st, w, X, ldx, M,
-                     per * 256, out, ldo, slab);
+// Waves of a workgroup: 4 up to 32 rows; 8 above, where half the staged activations per column count for more than a
+// second workgroup on the CU (28672 x 4096 Q4_K, 50 rows: 35 us against 47), and for the gated form, which has about
+// one workgroup a CU.
+template <int FMT, int MT, bool GLU>
+static void launch_skinny_t(const QW& w, const bf16* X, int ldx, int M, int splits, float* out, int ldo, long slab,
+                            const SkGlu& glu, hipStream_t st) {
+  constexpr int WV = GLU ? 8 : MT == 4 ? 8 : 4;
+  const int cols = GLU ? 64 : 16 * WV;
+  dim3 grid(((GLU ? glu.F : w.N) + cols - 1) / cols, splits);
+  hipLaunchKernelGGL((qgemm_skinny_kernel<FMT, MT, WV, GLU>), grid, dim3(64 * WV), 0, st, w, X, ldx, M,
+                     w.K / splits, out, ldo, slab, glu);
 }
 
-template <int FMT>
-static void launch_skinny_f(const QW& w, const bf16* X, int ldx, int M, int splits, float* out, int ldo,
-                            long slab, hipStream_t st) {
-  if (M <= 16) launch_skinny_t<FMT, 1>(w, X, ldx, M, splits, out, ldo, slab, st);
-  else if (M <= 32) launch_skinny_t<FMT, 2>(w, X, ldx, M, splits, out, ldo, slab, st);
-  else launch_skinny_t<FMT, 4>(w, X, ldx, M, splits, out, ldo, slab, st);
+template <int FMT, bool GLU>
+static void launch_skinny_f(const QW& w, const bf16* X, int ldx, int M, int splits, float* out, int ldo, long slab,
+                            const SkGlu& glu, hipStream_t st) {
+  if (M <= 16) launch_skinny_t<FMT, 1, GLU>(w, X, ldx, M, splits, out, ldo, slab, glu, st);
+  else if (M <= 32) launch_skinny_t<FMT, 2, GLU>(w, X, ldx, M, splits, out, ldo, slab, glu, st);
+  else launch_skinny_t<FMT, 4, GLU>(w, X, ldx, M, splits, out, ldo, slab, glu, st);
 }
 
 }  // namespace la
@@ -145,15 +428,40 @@ extern "C" int la_qgemm_skinny(int fmt, const void* p0, const void* p1, const vo
                                int ldo, long slab, void* stream) {
   using namespace la;
   if (M < 1 || M > 64 || (K & 255) || splits < 1 || ((K >> 8) % splits) || ldo < N || slab < (long)M * ldo) return -1;
+  if (fmt == FMT_Q6_K && (N & 1) && ((K >> 8) & 1)) return -1;   // SkW<FMT_Q6_K>: whole dwords of the plane of d
   QW w{(const uint8_t*)p0, (const uint8_t*)p1, (const uint8_t*)p2, (const uint8_t*)p3, N, K};
   hipStream_t st = (hipStream_t)stream;
   const bf16* x = (const bf16*)X;
   float* o = (float*)out;
   switch (fmt) {
-    case FMT_Q4_K: launch_skinny_f<FMT_Q4_K>(w, x, ldx, M, splits, o, ldo, slab, st); break;
-    case FMT_Q6_K: launch_skinny_f<FMT_Q6_K>(w, x, ldx, M, splits, o, ldo, slab, st); break;
-    case FMT_Q8_0: launch_skinny_f<FMT_Q8_0>(w, x, ldx, M, splits, o, ldo, slab, st); break;
-    case FMT_BF16: launch_skinny_f<FMT_BF16>(w, x, ldx, M, splits, o, ldo, slab, st); break;
+    case FMT_Q4_K: launch_skinny_f<FMT_Q4_K, false>(w, x, ldx, M, splits, o, ldo, slab, SkGlu{}, st); break;
+    case FMT_Q6_K: launch_skinny_f<FMT_Q6_K, false>(w, x, ldx, M, splits, o, ldo, slab, SkGlu{}, st); break;
+    case FMT_Q8_0: launch_skinny_f<FMT_Q8_0, false>(w, x, ldx, M, splits, o, ldo, slab, SkGlu{}, st); break;
+    case FMT_BF16: launch_skinny_f<FMT_BF16, false>(w, x, ldx, M, splits, o, ldo, slab, SkGlu{}, st); break;
+    default: return -2;
+  }
+  return (int)hipGetLastError();
+}
+
+// h = act(x Wg^T) * (x Wu^T) -> bf16 [M][ldo], F columns.  Gate rows oa .. oa + F of planes a, up rows ob .. ob + F of
+// planes b (the same planes with ob = F for one fused [2 F, K] weight).  act: 0 SwiGLU, 3 GeGLU (ops.ACT_*).
+extern "C" int la_qgemm_skinny_glu(int fmt, const void* const* a, int oa, const void* const* b, int ob, int F, int K,
+                                   const void* X, int ldx, int M, void* out, int ldo, int act, void* stream) {
+  using namespace la;
+  if (M < 1 || M > 64 || F < 1 || (K & 255) || ldo < F || ldx < K || (ldx & 7) || (act != 0 && act != 3)) return -1;
+  if (fmt == FMT_Q6_K && ((K >> 8) & 1) && (((oa + F) & 1) || ((ob + F) & 1))) return -1;   // whole dwords of the plane of d
+  auto qw = [K](const void* const* p, int n) {
+    return QW{(const uint8_t*)p[0], (const uint8_t*)p[1], (const uint8_t*)p[2], (const uint8_t*)p[3], n, K};
+  };
+  QW w = qw(a, oa + F);
+  const SkGlu glu{qw(b, ob + F), oa, ob, F, act, (bf16*)out};
+  hipStream_t st = (hipStream_t)stream;
+  const bf16* x = (const bf16*)X;
+  switch (fmt) {
+    case FMT_Q4_K: launch_skinny_f<FMT_Q4_K, true>(w, x, ldx, M, 1, nullptr, ldo, 0, glu, st); break;
+    case FMT_Q6_K: launch_skinny_f<FMT_Q6_K, true>(w, x, ldx, M, 1, nullptr, ldo, 0, glu, st); break;
+    case FMT_Q8_0: launch_skinny_f<FMT_Q8_0, true>(w, x, ldx, M, 1, nullptr, ldo, 0, glu, st); break;
+    case FMT_BF16: launch_skinny_f<FMT_BF16, true>(w, x, ldx, M, 1, nullptr, ldo, 0, glu, st); break;
     default: return -2;
   }
   return (int)hipGetLastError();

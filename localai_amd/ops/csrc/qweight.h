@@ -59,6 +59,28 @@ LA_DEV void q4k_scale_min(uint32_t a, uint32_t b, uint32_t c, int j, uint32_t& s
 
 template <int FMT> struct WFrag;
 
+// The forms below are written so that a weight costs one v_cvt_f32_ubyteN, one FMA and half a v_cvt_pk_bf16_f32 beside
+// the masks of its dword: the masked dword is opaque (otherwise hipcc extracts every nibble by itself, through SDWA,
+// and reorders the pairs with v_perm / v_alignbit: 36 instead of 23 instructions for 8 weights of Q4_K).
+LA_DEV uint32_t opaque(uint32_t v) {
+  asm("" : "+v"(v));
+  return v;
+}
+LA_DEV float ubyte_f(uint32_t v, int i) { return (float)((v >> (8 * i)) & 0xFFu); }
+LA_DEV uint32_t pk_bf16(float a, float b) {
+  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+  return __builtin_bit_cast(uint32_t, bf16x2{(bf16)a, (bf16)b});
+}
+// bf16 of s * byte + m for the 4 bytes of x and of y
+LA_DEV bf16x8 bytes_bf16(uint32_t x, uint32_t y, float s, float m) {
+  u32x4 r;
+  r.x = pk_bf16(fmaf(s, ubyte_f(x, 0), m), fmaf(s, ubyte_f(x, 1), m));
+  r.y = pk_bf16(fmaf(s, ubyte_f(x, 2), m), fmaf(s, ubyte_f(x, 3), m));
+  r.z = pk_bf16(fmaf(s, ubyte_f(y, 0), m), fmaf(s, ubyte_f(y, 1), m));
+  r.w = pk_bf16(fmaf(s, ubyte_f(y, 2), m), fmaf(s, ubyte_f(y, 3), m));
+  return __builtin_bit_cast(bf16x8, r);
+}
+
 // ---------------------------------------------------------------- Q4_K
 template <> struct WFrag<FMT_Q4_K> {
   u32x4 q0, q1, hdr;
@@ -84,15 +106,7 @@ template <> struct WFrag<FMT_Q4_K> {
     constexpr int h = S >> 2, t = S & 3;
     const uint32_t lo = (t == 0) ? q0.x : (t == 1) ? q0.z : (t == 2) ? q1.x : q1.z;
     const uint32_t hi = (t == 0) ? q0.y : (t == 1) ? q0.w : (t == 2) ? q1.y : q1.w;
-    const uint32_t a = (lo >> (4 * h)) & 0x0F0F0F0Fu, b = (hi >> (4 * h)) & 0x0F0F0F0Fu;
-    const float Dv = D[h], Mv = -Mn[h];
-    bf16x8 r;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      r[j] = (bf16)fmaf(Dv, (float)((a >> (8 * j)) & 0xFu), Mv);
-      r[j + 4] = (bf16)fmaf(Dv, (float)((b >> (8 * j)) & 0xFu), Mv);
-    }
-    return r;
+    return bytes_bf16(opaque((lo >> (4 * h)) & 0x0F0F0F0Fu), opaque((hi >> (4 * h)) & 0x0F0F0F0Fu), D[h], -Mn[h]);
   }
 };
 
@@ -129,16 +143,9 @@ template <> struct WFrag<FMT_Q6_K> {
     const uint32_t l0 = jh ? L.z : L.x, l1 = jh ? L.w : L.y;
     const uint32_t h0 = jh ? qh.z : qh.x, h1 = jh ? qh.w : qh.y;
     constexpr int ls = 4 * (qi >> 1), hs = 2 * qi;
-    const float sc = S[qi];
-    bf16x8 r;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      int q0 = (int)(((l0 >> (8 * j + ls)) & 0xFu) | (((h0 >> (8 * j + hs)) & 3u) << 4)) - 32;
-      int q1 = (int)(((l1 >> (8 * j + ls)) & 0xFu) | (((h1 >> (8 * j + hs)) & 3u) << 4)) - 32;
-      r[j] = (bf16)(sc * (float)q0);
-      r[j + 4] = (bf16)(sc * (float)q1);
-    }
-    return r;
+    const uint32_t u0 = opaque(((l0 >> ls) & 0x0F0F0F0Fu) | (((h0 >> hs) & 0x03030303u) << 4));
+    const uint32_t u1 = opaque(((l1 >> ls) & 0x0F0F0F0Fu) | (((h1 >> hs) & 0x03030303u) << 4));
+    return bytes_bf16(u0, u1, S[qi], -32.f * S[qi]);
   }
 };
 
@@ -165,14 +172,8 @@ template <> struct WFrag<FMT_Q8_0> {
     // bytes [32h + 8t, +8) of the lane's 64 bytes
     const u32x4& A = (h == 0) ? ((t < 2) ? a0 : a1) : ((t < 2) ? a2 : a3);
     const uint32_t lo = (t & 1) ? A.z : A.x, hi = (t & 1) ? A.w : A.y;
-    const float dv = d[h];
-    bf16x8 r;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      r[j] = (bf16)(dv * (float)(int8_t)((lo >> (8 * j)) & 0xFFu));
-      r[j + 4] = (bf16)(dv * (float)(int8_t)((hi >> (8 * j)) & 0xFFu));
-    }
-    return r;
+    // signed bytes with the sign bit flipped: 0 .. 255, 128 too much
+    return bytes_bf16(opaque(lo ^ 0x80808080u), opaque(hi ^ 0x80808080u), d[h], -128.f * d[h]);
   }
 };
 

@@ -6,6 +6,7 @@ import pytest
 import torch
 
 from localai_amd import ops
+from localai_amd.gguf import GGMLType, quantize
 
 pytestmark = pytest.mark.gpu
 DEV = torch.device("cuda:0")
@@ -56,3 +57,41 @@ def test_prefill_flash(Hq, Hkv, Dh, BS, qlens, ctx):
         ref = torch.einsum("hqk,khd->qhd", torch.softmax(sc.masked_fill(late, -math.inf), -1), v)
         assert (out[at:at + n] - ref).abs().max().item() <= 2 ** -7 * v.abs().max().item()
         at += n
+
+
+def _weight(N, K, t, seed):
+    w = np.random.default_rng(seed).standard_normal((N, K)).astype(np.float32) * 0.05
+    return ops.QWeight.from_raw(quantize(w, t), t, (N, K), DEV, keep_ref=True)
+
+
+SKINNY = [(GGMLType.Q4_K, 64, 256), (GGMLType.Q4_K, 200, 2816), (GGMLType.Q6_K, 130, 768), (GGMLType.Q6_K, 321, 1024),
+          (GGMLType.Q8_0, 72, 1280), (GGMLType.F16, 80, 512)]
+
+
+@pytest.mark.parametrize("t,N,K", SKINNY)
+@pytest.mark.parametrize("M", [3, 16, 17, 33, 64])
+def test_skinny_products(t, N, K, M):
+    """Fewer stages than ring slots, rows and columns past the last tile, an odd number of super-blocks, scales that
+    straddle dwords.  The weights are rounded to bf16 (2^-9 of each), the sums are fp32."""
+    w = _weight(N, K, t, N + K)
+    x = torch.randn(M, K, generator=torch.Generator().manual_seed(M)).to(torch.bfloat16)
+    y = ops.linear(x.to(DEV), w, force="skinny").dense().cpu()
+    bound = 2 ** -9 * (x.float().abs() @ w.ref.abs().t())
+    assert ((y - x.float() @ w.ref.t()).abs() <= bound + 1e-5).all()
+
+
+@pytest.mark.parametrize("t,N,K", SKINNY)
+@pytest.mark.parametrize("M,mode", [(3, ops.ACT_SWIGLU), (16, ops.ACT_GEGLU), (31, ops.ACT_SWIGLU), (64, ops.ACT_GEGLU)])
+def test_skinny_gated(t, N, K, M, mode):
+    """act(gate) * up in the product's epilogue, of two weights and of the halves of one: each product is off by at most
+    2^-9 of the sum of its terms' sizes, both activations' slopes stay below 1.2, the result is rounded to bf16."""
+    N &= ~15
+    a, b = _weight(N, K, t, 1), _weight(N, K, t, 2)
+    x = torch.randn(M, K, generator=torch.Generator().manual_seed(M)).to(torch.bfloat16)
+    g, u = x.float() @ a.ref.t(), x.float() @ b.ref.t()
+    eg, eu = (2 ** -9 * (x.float().abs() @ w.ref.abs().t()) for w in (a, b))
+    s = torch.nn.functional.silu(g) if mode == ops.ACT_SWIGLU else torch.nn.functional.gelu(g, approximate="tanh")
+    bound = 1.2 * eg * (u.abs() + eu) + s.abs() * eu + 2 ** -8 * (s * u).abs() + 1e-5
+    for ws in ([a, b], [ops.concat_rows([a, b])]):
+        h = ops.glu_linear(x.to(DEV), ws, N, mode)
+        assert h is not None and ((h.float().cpu() - s * u).abs() <= bound).all()
