@@ -51,7 +51,7 @@ constexpr int DEC_ONE_PART = 256;  // sequences up to this many keys run as a si
 
 template <int DH, int GT, int NW>
 struct DecShared {
-  float ow[NW < 2 ? 2 : NW][GT][DH];  // wave partials (NW > 1); the split-KV merge weights reuse it
+  float ow[NW < 2 ? 2 : NW][GT][DH];  // wave partials (NW > 1); the split-KV merge weights (65 GT) reuse it
   float mw[NW][16], lw[NW][16];
   int bt[DEC_MAXBT];
   int last;
@@ -137,6 +137,9 @@ LA_DEV float gate_at(const DecExtra& E, long row, int col) {
   return 1.f / (1.f + __expf(-(float)E.gate[row * E.ldg + col]));
 }
 
+LA_DEV void part_store(float* p, float v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+LA_DEV float part_load(const float* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+
 // K/V are streamed once per decode step: non-temporal loads (the default) read them 12-14 %
 // faster at batch 256 (5.05 -> 5.70 TB/s at 256 keys, 5.21 -> 5.98 at 384;
 // profiles/r4_attn_decode_nt.md).  VAR bit 0 = ordinary cached loads (A/B only); bit 1 = keys
@@ -154,7 +157,9 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2))) vo
   constexpr int NT = NW * 64;
   __shared__ DecShared<DH, GT, NW> sh;
 
-  const int p = blockIdx.x, kvh = blockIdx.y, b = blockIdx.z;
+  // kv heads fastest, partitions slowest: workgroups go to the XCDs in turn, and with the partitions fastest all first
+  // partitions of short sequences met on the same ones (8 x 200 keys, 32 partitions: 39 us instead of 12)
+  const int p = blockIdx.z, kvh = blockIdx.x, b = blockIdx.y;
   const int Hq = Hkv * G;
   const int L = seq_lens[b];
   // The grid's partitioning is fixed when a decode graph is captured (for the context bound);
@@ -164,7 +169,11 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2))) vo
   int wlo = window > 0 ? L - window : 0;  // first key inside the sliding window / the chunk
   if (E.chunk > 0) wlo = max(wlo, (L - 1) / E.chunk * E.chunk);
   const int base = wlo > 0 ? wlo / BS * BS : 0;  // partitions start at the page of the first visible key
-  const int PS = (L - base <= one_part && PS_grid < one_part) ? one_part : PS_grid;
+  // ... and of a longer one all P partitions take equal shares, in whole rounds of the waves (the context bound may
+  // be many times the sequence: shares of the bound would leave most of the grid without keys)
+  const int span = L - base, round = max(32 * NW, BS);
+  const int share = ((span + P - 1) / P + round - 1) / round * round;
+  const int PS = span <= one_part && PS_grid < one_part ? one_part : min(share, PS_grid);
   const int t0 = base + p * PS;
   if (t0 >= L) return;  // empty partition: the combiner only waits for ceil((L - base) / PS) of them
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -415,11 +424,11 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2))) vo
           }
         } else {
 #pragma unroll
-          for (int nd = 0; nd < ND; ++nd) part_o[(((long)b * Hq + hq) * P + p) * DH + 16 * nd + r] = o[nd][i];
+          for (int nd = 0; nd < ND; ++nd) part_store(part_o + (((long)b * Hq + hq) * P + p) * DH + 16 * nd + r, o[nd][i]);
           if (r == 0) {
             float* ml = part_ml + (((long)b * Hq + hq) * P + p) * 2;
-            ml[0] = mh;
-            ml[1] = lh;
+            part_store(ml, mh);
+            part_store(ml + 1, lh);
           }
         }
       }
@@ -454,66 +463,68 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2))) vo
       const float gf = E.gate ? gate_at(E, b, hq * DH + d) : 1.f;
       out[((long)b * Hq + hq) * DH + d] = (bf16)(den > 0.f ? num / den * gf : 0.f);
     } else {
-      part_o[(((long)b * Hq + hq) * P + p) * DH + d] = num;
+      part_store(part_o + (((long)b * Hq + hq) * P + p) * DH + d, num);
       if (d == 0) {
         float* ml = part_ml + (((long)b * Hq + hq) * P + p) * 2;
-        ml[0] = M;
-        ml[1] = den;
+        part_store(ml, M);
+        part_store(ml + 1, den);
       }
     }
   }
   if (np == 1) return;
   }
-  // ---- split-KV merge by the last-arriving partition of (b, kvh)
+  // ---- split-KV merge by the last-arriving partition of (b, kvh).  The partials are stored and loaded as relaxed
+  // agent-scope atomics, which go past the XCD's L2 by themselves: a release / acquire pair would write back and
+  // invalidate all of it.  Every thread's stores are complete before the barrier, and so before the ticket.
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
   if (tid == 0) {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     int* tk = tickets + (long)b * Hkv + kvh;
     const int prev = __hip_atomic_fetch_add(tk, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     const int last = (prev == np - 1);
-    if (last) {
-      *tk = 0;  // self-resetting ticket (next launch / graph replay starts from 0)
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    }
+    // self-resetting ticket (next launch / graph replay starts from 0)
+    if (last) __hip_atomic_store(tk, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     sh.last = last;
   }
   __syncthreads();
   if (!sh.last) return;
-  // merge weights per (partition, head) staged in LDS (reuses the wave-merge arrays), then every
-  // (head, d) output sums its np partials with independent, unrolled loads
+  // merge weights per (partition, head) staged in LDS (reuses the wave-merge arrays): a wave per head, a lane per
+  // partition (P <= 64), so the partials' maxima and sums cost one round trip
   float* wts = &sh.ow[0][0][0];  // [np][G] weights, then [G] 1/den
   const long hb = ((long)b * Hq + kvh * G) * P;
-  if (tid < G) {
-    const long base = hb + (long)tid * P;
-    float M = -INFINITY;
-    for (int j = 0; j < np; ++j) M = fmaxf(M, part_ml[(base + j) * 2]);
-    const float Ms = (M == -INFINITY) ? 0.f : M;
-    float den = 0.f;
-    for (int j = 0; j < np; ++j) {
-      const float f = exp2f(part_ml[(base + j) * 2] - Ms);
-      wts[j * G + tid] = f;
-      den += f * part_ml[(base + j) * 2 + 1];
-    }
-    wts[np * G + tid] = den > 0.f ? 1.f / den : 0.f;
+  for (int h = wave; h < G; h += NW) {
+    const float* ml = part_ml + (hb + (long)h * P + min(lane, np - 1)) * 2;
+    const float mj = part_load(ml), lj = part_load(ml + 1);
+    const float M = wave_max(lane < np ? mj : -INFINITY);
+    const float f = lane < np ? exp2f(mj - (M == -INFINITY ? 0.f : M)) : 0.f;
+    const float den = wave_sum(lane < np ? f * lj : 0.f);
+    if (lane < np) wts[lane * G + h] = f;
+    if (lane == 0) wts[np * G + h] = den > 0.f ? 1.f / den : 0.f;
   }
   __syncthreads();
-  for (int i = tid; i < G * DH; i += NT) {
+  // every pair of outputs sums its np partials, 16 loads of two in flight
+  for (int i = 2 * tid; i < G * DH; i += 2 * NT) {
     const int h = i / DH, d = i % DH;
-    const float* po = part_o + (hb + (long)h * P) * DH + d;
-    float num = 0.f;
-    for (int j0 = 0; j0 < np; j0 += 8) {
-      float v[8];
+    const uint64_t* po = (const uint64_t*)(part_o + (hb + (long)h * P) * DH + d);
+    float num[2] = {0.f, 0.f};
+    for (int j0 = 0; j0 < np; j0 += 16) {
+      uint64_t v[16];
 #pragma unroll
-      for (int j = 0; j < 8; ++j) v[j] = po[(long)min(j0 + j, np - 1) * DH];
+      for (int j = 0; j < 16; ++j)
+        v[j] = __hip_atomic_load(po + (long)min(j0 + j, np - 1) * (DH / 2), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 #pragma unroll
-      for (int j = 0; j < 8; ++j)
-        if (j0 + j < np) num += wts[(j0 + j) * G + h] * v[j];
+      for (int j = 0; j < 16; ++j)
+        if (j0 + j < np) {
+          const float f = wts[(j0 + j) * G + h];
+          num[0] += f * __uint_as_float((uint32_t)v[j]);
+          num[1] += f * __uint_as_float((uint32_t)(v[j] >> 32));
+        }
     }
-    const float gf = E.gate ? gate_at(E, b, (kvh * G + h) * DH + d) : 1.f;
-    out[((long)b * Hq + kvh * G + h) * DH + d] = (bf16)(num * wts[np * G + h] * gf);
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      const float gf = E.gate ? gate_at(E, b, (kvh * G + h) * DH + d + k) : 1.f;
+      out[((long)b * Hq + kvh * G + h) * DH + d + k] = (bf16)(num[k] * wts[np * G + h] * gf);
+    }
   }
 }
 
@@ -754,7 +765,7 @@ extern "C" int la_attn_decode(const void* q, const void* kc, const void* vc, con
   const la::DecExtra E{dist_bias, nbias, sink, sig, chunk, (const bf16*)gate, ldg, keep};
   const int G = Hq / Hkv;
   hipStream_t st = (hipStream_t)stream;
-  dim3 grid(P, Hkv, B);
+  dim3 grid(Hkv, B, P);
   float* po = (float*)part_o;
   float* pml = (float*)part_ml;
   int* tk = (int*)tickets;

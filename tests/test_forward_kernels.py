@@ -95,3 +95,24 @@ def test_skinny_gated(t, N, K, M, mode):
     for ws in ([a, b], [ops.concat_rows([a, b])]):
         h = ops.glu_linear(x.to(DEV), ws, N, mode)
         assert h is not None and ((h.float().cpu() - s * u).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("Hq,Hkv,Dh,BS,lens,bound", [(32, 8, 128, 32, [8001], 16384), (8, 8, 128, 16, [1, 128, 129, 256, 257, 385, 2049], 4096),
+                                                     (16, 1, 64, 64, [255, 700, 5000], 5000), (12, 4, 80, 32, [1000] * 20, 4096)])
+def test_decode_shares(Hq, Hkv, Dh, BS, lens, bound):
+    """Partitions are equal shares of each sequence's own keys: one, up to all 64, and lengths at the edges of a round
+    of the waves; twice in a row, as the tickets reset themselves.  Weights and result are rounded to bf16 as in the
+    prompt kernel.  (Places without a key are zero: this kernel multiplies them by a weight of 0.)"""
+    kc, vc, bt, keys, values = _pages(lens, Hkv, Dh, BS, seed=len(lens))
+    kc, vc = kc.nan_to_num(), vc.nan_to_num()
+    q = torch.randn(len(lens), Hq, Dh, generator=torch.Generator().manual_seed(3)).to(torch.bfloat16)
+    args = [t.to(DEV) for t in (q, kc, vc, bt, torch.tensor(lens, dtype=torch.int32))]
+    ws = ops.decode_workspace(len(lens), Hq, Hkv, Dh, bound, DEV, BS)
+    first = ops.attn_decode(*args, 1 / math.sqrt(Dh), bound, workspace=ws).cpu()
+    again = ops.attn_decode(*args, 1 / math.sqrt(Dh), bound, workspace=ws).cpu()
+    assert torch.equal(first, again)
+    for s, n in enumerate(lens):
+        k, v = (x[s].repeat_interleave(Hq // Hkv, 1) for x in (keys, values))
+        w = torch.softmax(torch.einsum("hd,khd->hk", q[s].float(), k) / math.sqrt(Dh), -1)
+        ref = torch.einsum("hk,khd->hd", w, v)
+        assert (first[s].float() - ref).abs().max().item() <= 2 ** -7 * v.abs().max().item()
