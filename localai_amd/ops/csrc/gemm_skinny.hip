@@ -268,12 +268,12 @@ struct SkCfg {
   static constexpr int FIT = (160 * 1024 - QUADS) / SLOT;
   static constexpr int NS = WANT >= 4 ? (WANT > 8 ? 8 : WANT) : FIT < 4 ? FIT : 4;
   static_assert(NS >= 3, "ring");
+  static constexpr int LDS = NS * SLOT + QUADS;
 };
 
 template <int FMT, int MT, int WV, bool GLU>
-__global__ __launch_bounds__(64 * WV, 2) void qgemm_skinny_kernel(
-    QW w, const bf16* __restrict__ X, int ldx, int M, int k_per_split, float* __restrict__ out, int ldo,
-    long slab, SkGlu glu) {
+LA_DEV void sk_tile(uint8_t* lds, const QW& w, int tile, const bf16* __restrict__ X, int ldx, int M, int k_per_split,
+                    float* __restrict__ out, int ldo, long slab, const SkGlu& glu) {
   static_assert(!GLU || WV == 8, "4 waves of gate and 4 of up tiles");
   using W = SkW<FMT>;
   using C = SkCfg<FMT, MT, WV, GLU>;
@@ -281,14 +281,13 @@ __global__ __launch_bounds__(64 * WV, 2) void qgemm_skinny_kernel(
   constexpr int PX = 4 * MT < WV ? 1 : 4 * MT / WV;    // pieces (4 rows) of X a wave fetches; MT 1, 8 waves: each by two
   constexpr int L = PX + W::PIECES;                    // DMAs of a wave per stage
   static_assert((NS - 3) * L < 64 && NS <= 8, "vmcnt; a quad's scales have landed 8 stages later");
-  __shared__ __attribute__((aligned(1024))) uint8_t lds[NS * C::SLOT + C::QUADS];
 
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int g = lane >> 4, r = lane & 15;
   const int N = GLU ? glu.F : w.N;
   const int nst = k_per_split / SK_K, ks0 = blockIdx.y * nst;
   const bool up = GLU && wave >= 4;
-  const int c0 = GLU ? (blockIdx.x * 4 + (wave & 3)) * 16 : (blockIdx.x * WV + wave) * 16;   // the wave's first column
+  const int c0 = GLU ? (tile * 4 + (wave & 3)) * 16 : (tile * WV + wave) * 16;   // the wave's first column
 
   // sources: pieces of X, the tile's planes (rows past N repeat the last)
   const bf16* xp[PX];
@@ -399,6 +398,27 @@ __global__ __launch_bounds__(64 * WV, 2) void qgemm_skinny_kernel(
   }
 }
 
+template <int FMT, int MT, int WV, bool GLU>
+__global__ __launch_bounds__(64 * WV, 2) void qgemm_skinny_kernel(
+    QW w, const bf16* __restrict__ X, int ldx, int M, int k_per_split, float* __restrict__ out, int ldo,
+    long slab, SkGlu glu) {
+  __shared__ __attribute__((aligned(1024))) uint8_t lds[SkCfg<FMT, MT, WV, GLU>::LDS];
+  sk_tile<FMT, MT, WV, GLU>(lds, w, blockIdx.x, X, ldx, M, k_per_split, out, ldo, slab, glu);
+}
+
+// Two weights of the same K and different formats side by side (q|k in Q4_K beside v in Q6_K): columns 0 .. wa.N of
+// the output from the first tiles_a workgroups of every split, the others from the rest.  v alone is 16 workgroups.
+template <int FA, int FB, int MT, int WV>
+__global__ __launch_bounds__(64 * WV, 2) void qgemm_skinny2_kernel(
+    QW wa, QW wb, int tiles_a, const bf16* __restrict__ X, int ldx, int M, int k_per_split, float* __restrict__ out,
+    int ldo, long slab) {
+  constexpr int LA = SkCfg<FA, MT, WV, false>::LDS, LB = SkCfg<FB, MT, WV, false>::LDS;
+  __shared__ __attribute__((aligned(1024))) uint8_t lds[LA > LB ? LA : LB];
+  const int t = blockIdx.x;
+  if (t < tiles_a) sk_tile<FA, MT, WV, false>(lds, wa, t, X, ldx, M, k_per_split, out, ldo, slab, SkGlu{});
+  else sk_tile<FB, MT, WV, false>(lds, wb, t - tiles_a, X, ldx, M, k_per_split, out + wa.N, ldo, slab, SkGlu{});
+}
+
 // Waves of a workgroup: 4 up to 32 rows; 8 above, where half the staged activations per column count for more than a
 // second workgroup on the CU (28672 x 4096 Q4_K, 50 rows: 35 us against 47), and for the gated form, which has about
 // one workgroup a CU.
@@ -418,6 +438,14 @@ static void launch_skinny_f(const QW& w, const bf16* X, int ldx, int M, int spli
   if (M <= 16) launch_skinny_t<FMT, 1, GLU>(w, X, ldx, M, splits, out, ldo, slab, glu, st);
   else if (M <= 32) launch_skinny_t<FMT, 2, GLU>(w, X, ldx, M, splits, out, ldo, slab, glu, st);
   else launch_skinny_t<FMT, 4, GLU>(w, X, ldx, M, splits, out, ldo, slab, glu, st);
+}
+
+template <int FA, int FB, int MT, int WV>
+static void launch_skinny2(const QW& wa, const QW& wb, const bf16* X, int ldx, int M, int splits, float* out, int ldo,
+                           long slab, hipStream_t st) {
+  const int cols = 16 * WV, ta = (wa.N + cols - 1) / cols, tb = (wb.N + cols - 1) / cols;
+  hipLaunchKernelGGL((qgemm_skinny2_kernel<FA, FB, MT, WV>), dim3(ta + tb, splits), dim3(64 * WV), 0, st, wa, wb, ta, X,
+                     ldx, M, wa.K / splits, out, ldo, slab);
 }
 
 }  // namespace la
@@ -464,5 +492,24 @@ extern "C" int la_qgemm_skinny_glu(int fmt, const void* const* a, int oa, const 
     case FMT_BF16: launch_skinny_f<FMT_BF16, true>(w, x, ldx, M, 1, nullptr, ldo, 0, glu, st); break;
     default: return -2;
   }
+  return (int)hipGetLastError();
+}
+
+// [x Wa^T | x Wb^T] of a Q4_K and a Q6_K weight of the same K in one launch: fp32 slabs [splits][M][ldo].
+extern "C" int la_qgemm_skinny2(const void* const* a, int Na, const void* const* b, int Nb, int K, const void* X, int ldx,
+                                int M, int splits, void* out, int ldo, long slab, void* stream) {
+  using namespace la;
+  if (M < 1 || M > 64 || Na < 1 || Nb < 1 || (K & 255) || splits < 1 || ((K >> 8) % splits) || ldo < Na + Nb ||
+      slab < (long)M * ldo || ldx < K || (ldx & 7))
+    return -1;
+  if ((Nb & 1) && ((K >> 8) & 1)) return -1;   // SkW<FMT_Q6_K>: whole dwords of the plane of d
+  const QW wa{(const uint8_t*)a[0], (const uint8_t*)a[1], (const uint8_t*)a[2], (const uint8_t*)a[3], Na, K};
+  const QW wb{(const uint8_t*)b[0], (const uint8_t*)b[1], (const uint8_t*)b[2], (const uint8_t*)b[3], Nb, K};
+  hipStream_t st = (hipStream_t)stream;
+  const bf16* x = (const bf16*)X;
+  float* o = (float*)out;
+  if (M <= 16) launch_skinny2<FMT_Q4_K, FMT_Q6_K, 1, 4>(wa, wb, x, ldx, M, splits, o, ldo, slab, st);
+  else if (M <= 32) launch_skinny2<FMT_Q4_K, FMT_Q6_K, 2, 4>(wa, wb, x, ldx, M, splits, o, ldo, slab, st);
+  else launch_skinny2<FMT_Q4_K, FMT_Q6_K, 4, 8>(wa, wb, x, ldx, M, splits, o, ldo, slab, st);
   return (int)hipGetLastError();
 }

@@ -116,3 +116,18 @@ def test_decode_shares(Hq, Hkv, Dh, BS, lens, bound):
         w = torch.softmax(torch.einsum("hd,khd->hk", q[s].float(), k) / math.sqrt(Dh), -1)
         ref = torch.einsum("hk,khd->hd", w, v)
         assert (first[s].float() - ref).abs().max().item() <= 2 ** -7 * v.abs().max().item()
+
+
+@pytest.mark.parametrize("M", [3, 17, 64])
+@pytest.mark.parametrize("Na,Nb,K", [(320, 64, 1024), (130, 71, 512), (64, 200, 2816)])
+def test_skinny_pair(M, Na, Nb, K):
+    """A Q4_K and a Q6_K weight side by side in one launch against each alone: the same sums, bit for bit."""
+    ws = [_weight(Na, K, GGMLType.Q4_K, 1), _weight(Nb, K, GGMLType.Q6_K, 2)]
+    x = torch.randn(M, K, generator=torch.Generator().manual_seed(M)).to(torch.bfloat16).to(DEV)
+    y = ops.linear_multi(x, ws, force="skinny")
+    S = y.S
+    alone = [ops.linear(x, w, force="skinny", out_slabs=torch.empty(S, M, w.N, device=DEV)) for w in ws]
+    if all(p.S == S for p in alone):
+        assert torch.equal(y.t, torch.cat([p.t for p in alone], -1))
+    else:
+        assert torch.allclose(y.dense(), torch.cat([p.dense() for p in alone], -1), rtol=1e-5, atol=1e-5)
