@@ -66,6 +66,9 @@ def lib():
         P, I, F, LNG = ctypes.c_void_p, ctypes.c_int, ctypes.c_float, ctypes.c_long
         sig = {
             "la_qgemm_skinny": [I, P, P, P, P, I, I, P, I, I, I, P, I, LNG, P],
+            "la_wgemm": [I, P, I, I, P, I, I, I, P, I, LNG, I, I, P],
+            "la_wgemm2": [P, I, P, I, I, P, I, I, I, P, I, LNG, I, I, P],
+            "la_wgemm_glu": [I, P, I, P, I, I, I, P, I, I, P, I, I, I, P],
             "la_qgemm_skinny2": [P, I, P, I, I, P, I, I, I, P, I, LNG, P],
             "la_qgemm_skinny_glu": [I, P, I, P, I, I, I, P, I, I, P, I, I, P],
             "la_qgemv_dp4": [I, P, P, P, I, P, I, I, I, P, I, LNG, P, LNG, I, P, I, P],
@@ -961,6 +964,50 @@ def _run_bs_glu(x, pair, F: int, mode: int, var: int, out) -> None:
                                mode, var, _stream()), "la_bsgemm_glu")
 
 
+# Two-K-group GEMM (gemm_wide.hip): rb = rows of a workgroup / 64, 128 columns.
+W_FMTS = (FMT_Q4_K, FMT_Q6_K, FMT_Q8_0)
+
+
+def w_ok(ws: Sequence[QWeight]) -> bool:
+    """Can gemm_wide.hip run these weights (one launch per weight, or one for q|k in Q4_K beside v in Q6_K)."""
+    return _has("la_wgemm") and all(w.fmt in W_FMTS and w.planes[0] is not None and _skinny_ok(w) for w in ws)
+
+
+def _w_grid(M: int, N: int, rb: int) -> int:
+    return -(-M // (64 * rb)) * -(-N // 128)
+
+
+def _w_split_ok(K: int, S: int) -> bool:
+    return S >= 1 and -(-(K // 128) // S) * (S - 1) < K // 128
+
+
+def _planes4(w: QWeight):
+    return (ctypes.c_void_p * 4)(*w.ptrs())
+
+
+def _run_w(x, ws, S, out, Ntot, rb):
+    """out: fp32 slabs [S, M, Ntot], or a bf16 [M, Ntot] matrix (S == 1)."""
+    M, K = x.shape
+    bf = out.dtype == torch.bfloat16
+    slab = 0 if bf else M * Ntot
+    if len(ws) == 2 and (ws[0].fmt, ws[1].fmt) == (FMT_Q4_K, FMT_Q6_K):
+        _check(lib().la_wgemm2(_planes4(ws[0]), ws[0].N, _planes4(ws[1]), ws[1].N, K, x.data_ptr(), K, M, S, out.data_ptr(),
+                               Ntot, slab, int(bf), rb, _stream()), "la_wgemm2")
+        return
+    col = 0
+    for w in ws:
+        _check(lib().la_wgemm(w.fmt, _planes4(w), w.N, K, x.data_ptr(), K, M, S, out.data_ptr() + col * (2 if bf else 4),
+                              Ntot, slab, int(bf), rb, _stream()), "la_wgemm")
+        col += w.N
+
+
+def _run_w_glu(x, pair, F: int, mode: int, rb: int, out) -> None:
+    M, K = x.shape
+    wa, oa, wb, ob = pair
+    _check(lib().la_wgemm_glu(wa.fmt, _planes4(wa), oa, _planes4(wb), ob, F, K, x.data_ptr(), K, M, out.data_ptr(), F, mode,
+                              rb, _stream()), "la_wgemm_glu")
+
+
 def _q32_grid(M: int, N: int, var: int) -> int:
     bm, bn = Q32_TILES[var]
     return -(-M // bm) * -(-N // bn)
@@ -1019,6 +1066,12 @@ def _autotune_mid(x, ws, key, Ntot):
             for S in sorted({1, max(1, base // 2), base, base * 2}):
                 if S <= min(8, K // 256) and _tile_split_ok(K, S):
                     cands.append(("bs", S, v))
+    if w_ok(ws):
+        for rb in (4, 2) if M > 128 else (2,):
+            base = max(1, round(256 / _w_grid(M, Ntot, rb)))
+            for S in sorted({1, max(1, base // 2), base, base * 2}):
+                if S <= min(8, K // 256) and _w_split_ok(K, S):
+                    cands.append(("w", S, rb))
     if not cands or not TILE_GEMM:
         cands = [("blas", 0, 0)]
     outs = {S: torch.empty(S, M, Ntot, dtype=torch.float32, device=x.device) for _, S, _ in cands if S > 1}
@@ -1031,6 +1084,8 @@ def _autotune_mid(x, ws, key, Ntot):
             fn = lambda S=S, t=t: _run_tile(x, ws, S, outs[S], Ntot, t)  # noqa: E731
         elif kind == "bs":
             fn = lambda S=S, t=t: _run_bs(x, ws, S, outs[S], Ntot, t)  # noqa: E731
+        elif kind == "w":
+            fn = lambda S=S, t=t: _run_w(x, ws, S, outs[S], Ntot, t)  # noqa: E731
         else:
             fn = lambda S=S, t=t: _run_q32(x, ws, S, outs[S], Ntot, t)  # noqa: E731
         fn()
@@ -1051,6 +1106,62 @@ def _autotune_mid(x, ws, key, Ntot):
             best, best_t = (kind, S, t), tt
     _GEMM_CHOICE[key] = best
     return best
+
+
+# Time of one K step of a workgroup (us; a step is 64 k of a 256 x 256 tile, 128 k of a 256 x 128 one), chip full
+_STEP_US = {"tile": {FMT_Q4_K: 1.75, FMT_Q6_K: 2.05, FMT_Q8_0: 1.85}, "w": {FMT_Q4_K: 2.1, FMT_Q6_K: 2.4, FMT_Q8_0: 2.2}}
+QUANT_MAX_M = 1280
+
+
+@functools.lru_cache(maxsize=4096)
+def _quant_plan(M: int, K: int, ws: Tuple[Tuple[int, int], ...], glu: bool, tile_ok: bool, wide_ok: bool) -> Optional[tuple]:
+    """(kind, S, tile) of the product that reads the quantised weights ((fmt, N), ...) itself, or None where a bf16 copy
+    and the library's GEMM are faster: the rule for MID_MAX_M < M <= QUANT_MAX_M rows.  A rule and no autotuning, since
+    the length of a prompt chunk differs per call.
+
+    The library has to be paid the copy (N K weights written and read back, 2.56 B each at 4.2 TB/s), 10 us + K / 400
+    for its launches and its pipeline, and the product at 1.4 PF/s.  A product on the quantised weights costs whole
+    rounds of the 256 CUs and, split, 8 bytes of slab for each sum.  Measured with the consumer (us, plan against copy
+    + library), Q4_K: 4096 x 14336 at 288 rows 71 / 118, 512 84 / 124, 701 111 / 143, 1024 139 / 161, 1280 170 / 188,
+    1536 222 / 216; gate|up 28672 x 4096 at 400 rows 125 / 174, 701 208 / 229, 1024 250 / 267, 1280 348 / 342; 4096 x
+    4096 at 400 rows 37 / 42, 701 51 / 50.  Q6_K 4096 x 14336 at 512 rows 93 / 131, 701 126 / 148.  The estimates below
+    are within some 10 % of these, and within 15 % for 2048 to 28672 k and 2048 to 57344 columns."""
+    if not MID_MAX_M < M <= QUANT_MAX_M or any(f not in W_FMTS for f, _ in ws):
+        return None
+    N = sum(n for _, n in ws)
+    lib_us = 10 + K / 400 + N * K * 2.56 / 4.2e6 + 2 * M * N * K / 1.4e9
+    if glu:
+        lib_us += 3 + M * N * 3 / 4e6                    # the activation's own pass
+    best, best_us = None, 0.95 * lib_us
+    for kind, bn, bk, ok in (("tile", 256, 64, tile_ok), ("w", 128, 128, wide_ok)):
+        if not ok:
+            continue
+        step = max(_STEP_US[kind][f] for f, _ in ws) + (0.15 if glu and kind == "tile" else 0)
+        tiles = -(-M // 256) * sum(-(-n // bn) for _, n in ws)
+        for S in range(1, 2 if glu else 9):
+            if not (_tile_split_ok(K, S) if kind == "tile" else _w_split_ok(K, S)):
+                continue
+            us = -(-tiles * S // 256) * -(-(K // bk) // S) * step + 8 + (S * M * N * 8 / 4.5e6 if S > 1 else 0)
+            if us < best_us:
+                best, best_us = (kind, S, 6 if kind == "tile" else 4), us
+    return best
+
+
+def _plan_quant(M: int, K: int, ws: Sequence[QWeight], glu: bool = False) -> Optional[tuple]:
+    """_quant_plan for these weights, where what it needs is there.  The 256 x 256 tiles read a plane of scales that is
+    built once per weight (0.125 B each): not inside a capture, and only while 4 GiB of the card stay free."""
+    if not (MID_MAX_M < M <= QUANT_MAX_M and TILE_GEMM and PREFILL_GEMM == "blas") or any(w.bf16 is not None for w in ws):
+        return None
+    if not all(w.fmt in W_FMTS and w.tile_ok for w in ws) or len(ws) > 1 and (glu or (ws[0].fmt, ws[1].fmt, len(ws)) != (FMT_Q4_K, FMT_Q6_K, 2)):
+        return None
+    w = ws[0]
+    tile_ok = len(ws) == 1 and _has("la_qgemm_tile")
+    key = (M, K, tuple((w.fmt, w.N) for w in ws), glu)
+    plan = _quant_plan(*key, tile_ok, w_ok(ws))
+    if plan is not None and plan[0] == "tile" and w.gsc is None:
+        if torch.cuda.is_current_stream_capturing() or torch.cuda.mem_get_info(w.device)[0] < (4 << 30) + w.N * w.K // 8:
+            plan = _quant_plan(*key, False, w_ok(ws))
+    return plan
 
 
 def _skinny_ok(w: QWeight) -> bool:
@@ -1089,7 +1200,7 @@ def linear_multi(x: torch.Tensor, ws: Sequence[QWeight], bias: Optional[torch.Te
     use_skinny = (M <= SKINNY_MAX_M and skinny_ok) if force is None else force == "skinny"
     tile_ok = TILE_GEMM and all(w.tile_ok for w in ws) and (_has("la_qgemm_tile") or _has("la_qgemm32") or _has("la_bsgemm"))
     S, tile, kind = 0, 0, None
-    if force is not None and (force.startswith("q32:") or force.startswith("bs:")):
+    if force is not None and force.split(":")[0] in ("q32", "bs", "w"):
         kind, v, s_ = force.split(":")
         tile, S = int(v), int(s_)
     elif force is not None and force.startswith("tile"):
@@ -1107,14 +1218,18 @@ def linear_multi(x: torch.Tensor, ws: Sequence[QWeight], bias: Optional[torch.Te
         if choice is None and tile_ok and _has("la_qgemm_tile"):
             t, s_ = pick_tile(M, [w.N for w in ws], K)
             choice = ("tile", s_, t)
-        if choice is not None and choice[0] in ("tile", "q32", "bs"):
+        if choice is not None and choice[0] in ("tile", "q32", "bs", "w"):
             kind, S, tile = choice
     elif force is None and not use_skinny and tile_ok and PREFILL_GEMM == "tile":
         tile, S = pick_tile(M, [w.N for w in ws], K)   # prefill: heuristic, never tuned inline
         kind = "tile"
-    if kind in ("tile", "q32", "bs") and S == 1 and out_slabs is None:
+    elif force is None and not use_skinny:
+        plan = _plan_quant(M, K, ws)
+        if plan is not None:
+            kind, S, tile = plan
+    if kind in ("tile", "q32", "bs", "w") and S == 1 and out_slabs is None:
         y = torch.empty(M, Ntot, dtype=torch.bfloat16, device=x.device)
-        {"tile": _run_tile, "q32": _run_q32, "bs": _run_bs}[kind](x, ws, 1, y, Ntot, tile)
+        {"tile": _run_tile, "q32": _run_q32, "bs": _run_bs, "w": _run_w}[kind](x, ws, 1, y, Ntot, tile)
         return Partial(y, bias)
     if S:
         out = out_slabs
@@ -1124,6 +1239,8 @@ def linear_multi(x: torch.Tensor, ws: Sequence[QWeight], bias: Optional[torch.Te
             _run_tile(x, ws, S, out, Ntot, tile)
         elif kind == "bs":
             _run_bs(x, ws, S, out, Ntot, tile)
+        elif kind == "w":
+            _run_w(x, ws, S, out, Ntot, tile)
         else:
             _run_q32(x, ws, S, out, Ntot, tile)
         return Partial(out, bias)
@@ -1178,9 +1295,13 @@ def _glu_pair(ws: Sequence[QWeight], F: int):
 
 
 def _run_glu(x: torch.Tensor, pair, F: int, mode: int, tile: int, out: torch.Tensor) -> None:
-    """tile < 100: gemm_q.hip tile id; 100 + v: gemm_q32.hip variant v; 200 + v: gemm_bs.hip variant v."""
+    """tile < 100: gemm_q.hip tile id; 100 + v: gemm_q32.hip variant v; 200 + v: gemm_bs.hip variant v; 300 + rb:
+    gemm_wide.hip."""
     M, K = x.shape
     wa, oa, wb, ob = pair
+    if tile >= 300:
+        _run_w_glu(x, pair, F, mode, tile - 300, out)
+        return
     if tile >= 200:
         _run_bs_glu(x, pair, F, mode, tile - 200, out)
         return
@@ -1230,9 +1351,16 @@ def glu_linear(x: torch.Tensor, ws: Sequence[QWeight], F: int, mode: int,
         return None
     M, K = x.shape
     if M > MID_MAX_M:
-        # prefill chunks: dequant + hipBLASLt + the activation kernel beats every fused GLU tile
-        # at M >= 1024 (gemm_bs.hip's GLU mode included, profiles/r6_gemm_bs.md)
-        return None
+        # prompt chunks: a rule, never tuned inline (dequant + hipBLASLt + the activation kernel beats every fused GLU
+        # tile from 1280 rows on)
+        plan = _plan_quant(M, K, ws, True) if len(ws) == 1 and ws[0].N == 2 * F and _glu_pair(ws, F) else None
+        if plan is None:
+            return None
+        if x.dtype != torch.bfloat16 or not x.is_contiguous() or K != ws[0].K:
+            raise ValueError("glu_linear: x must be contiguous bf16 [M, K]")
+        out = torch.empty(M, F, dtype=torch.bfloat16, device=x.device)
+        _run_glu(x, _glu_pair(ws, F), F, mode, plan[2] if plan[0] == "tile" else 300 + plan[2], out)
+        return out
     pair = _glu_pair(ws, F)
     if pair is None:
         return None
@@ -1256,6 +1384,8 @@ def glu_linear(x: torch.Tensor, ws: Sequence[QWeight], F: int, mode: int,
             cands += [109, 108, 104] if M > 128 else [109, 108, 107]
         if bs_ok([pair[0], pair[2]]) and pair[0].fmt == pair[2].fmt and F % 4 == 0:
             cands += [200, 203] if M > 128 else [201]
+        if w_ok([pair[0], pair[2]]) and pair[0].fmt == pair[2].fmt:
+            cands += [304, 302] if M > 128 else [302]
         for t in cands:
             tt = _time_cold(lambda t=t: _run_glu(x, pair, F, mode, t, out))
             if tt < best_t:

@@ -131,3 +131,66 @@ def test_skinny_pair(M, Na, Nb, K):
         assert torch.equal(y.t, torch.cat([p.t for p in alone], -1))
     else:
         assert torch.allclose(y.dense(), torch.cat([p.dense() for p in alone], -1), rtol=1e-5, atol=1e-5)
+
+
+@pytest.mark.parametrize("t,N,K,S", [(GGMLType.Q4_K, 256, 256, 1), (GGMLType.Q4_K, 200, 2816, 3), (GGMLType.Q6_K, 130, 768, 1),
+                                     (GGMLType.Q6_K, 321, 1024, 2), (GGMLType.Q8_0, 72, 1280, 5), (GGMLType.Q8_0, 384, 4352, 4)])
+@pytest.mark.parametrize("M,rb", [(65, 2), (128, 2), (129, 4), (256, 4), (300, 4), (300, 2)])
+def test_wide_products(t, N, K, S, M, rb):
+    """Rows and columns past the last tile, splits that begin inside a quad of scales, a shorter last split, an odd
+    number of super-blocks; fp32 slabs and the bf16 matrix.  Bounds as for the skinny products, plus the result's
+    rounding."""
+    w = _weight(N, K, t, N + K)
+    x = torch.randn(M, K, generator=torch.Generator().manual_seed(M)).to(torch.bfloat16)
+    ref = x.float() @ w.ref.t()
+    bound = 2 ** -9 * (x.float().abs() @ w.ref.abs().t()) + 1e-5
+    slabs = torch.empty(S, M, N, device=DEV)
+    y = ops.linear(x.to(DEV), w, force=f"w:{rb}:{S}", out_slabs=slabs).dense().cpu()
+    assert ((y - ref).abs() <= bound).all()
+    y = ops.linear(x.to(DEV), w, force=f"w:{rb}:1").dense().cpu()
+    assert ((y - ref).abs() <= bound + 2 ** -8 * ref.abs()).all()
+
+
+@pytest.mark.parametrize("t", [GGMLType.Q4_K, GGMLType.Q6_K, GGMLType.Q8_0])
+@pytest.mark.parametrize("F,K,M,rb", [(64, 512, 65, 2), (80, 2816, 256, 4), (144, 256, 200, 4), (208, 1024, 128, 2)])
+def test_wide_gated(t, F, K, M, rb):
+    """The gated form against the plain products; bounds as for the skinny one."""
+    a, b = _weight(F, K, t, 1), _weight(F, K, t, 2)
+    x = torch.randn(M, K, generator=torch.Generator().manual_seed(M)).to(torch.bfloat16)
+    g, u = x.float() @ a.ref.t(), x.float() @ b.ref.t()
+    eg, eu = (2 ** -9 * (x.float().abs() @ w.ref.abs().t()) for w in (a, b))
+    s = torch.nn.functional.silu(g)
+    bound = 1.2 * eg * (u.abs() + eu) + s.abs() * eu + 2 ** -8 * (s * u).abs() + 1e-5
+    for pair in ((a, 0, b, 0), (ops.concat_rows([a, b]), 0, ops.concat_rows([a, b]), F)):
+        h = torch.empty(M, F, dtype=torch.bfloat16, device=DEV)
+        ops._run_glu(x.to(DEV), pair, F, ops.ACT_SWIGLU, 300 + rb, h)
+        assert ((h.float().cpu() - s * u).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("M,rb,S", [(70, 2, 2), (256, 4, 3), (256, 4, 1)])
+def test_wide_pair(M, rb, S):
+    """Q4_K and Q6_K side by side against each alone."""
+    ws = [_weight(200, 1536, GGMLType.Q4_K, 1), _weight(72, 1536, GGMLType.Q6_K, 2)]
+    x = torch.randn(M, 1536, generator=torch.Generator().manual_seed(M)).to(torch.bfloat16).to(DEV)
+    y = ops.linear_multi(x, ws, force=f"w:{rb}:{S}", out_slabs=torch.empty(S, M, 272, device=DEV))
+    alone = [ops.linear(x, w, force=f"w:{rb}:{S}", out_slabs=torch.empty(S, M, w.N, device=DEV)) for w in ws]
+    assert torch.equal(y.t, torch.cat([p.t for p in alone], -1))
+
+
+@pytest.mark.parametrize("t,N,K,M,kind", [(GGMLType.Q4_K, 2048, 8192, 257, "w"), (GGMLType.Q4_K, 2050, 8192, 512, "w"), (GGMLType.Q6_K, 4096, 14336, 701, "tile"),
+                                          (GGMLType.Q8_0, 4096, 14336, 1024, "tile"), (GGMLType.Q4_K, 4096, 4096, 1280, None)])
+def test_prompt_plan(t, N, K, M, kind):
+    """Either side of the line between the quantised products and the copy with the library's: same sums, and the gated
+    form through its entry.  Every path rounds a weight to bf16 and sums in fp32; the copy's result is rounded once more."""
+    w = _weight(N, K, t, N + K)
+    x = torch.randn(M, K, generator=torch.Generator().manual_seed(M)).to(torch.bfloat16).to(DEV)
+    plan = ops._plan_quant(M, K, [w])
+    assert (plan[0] if plan else None) == kind
+    wf = w.ref.to(DEV)
+    ref, bound = x.float() @ wf.t(), 2 ** -9 * (x.float().abs() @ wf.abs().t()) + 1e-4
+    assert ((ops.linear(x, w).dense() - ref).abs() <= bound + 2 ** -8 * ref.abs()).all()
+    h = ops.glu_linear(x, [w], N // 2, ops.ACT_SWIGLU)
+    if h is not None:
+        s, u = torch.nn.functional.silu(ref[:, :N // 2]), ref[:, N // 2:]
+        eg, eu = bound[:, :N // 2], bound[:, N // 2:]
+        assert ((h.float() - s * u).abs() <= 1.2 * eg * (u.abs() + eu) + s.abs() * eu + 2 ** -8 * (s * u).abs() + 1e-5).all()
