@@ -17,20 +17,35 @@
 //    16-byte read.
 //  * The second half of a step is multiplied beside the first dequantisation of the next (sched_group_barrier: six
 //    vector instructions after an MFMA), so neither waits for the other inside a wave.
-// What bounds it: the dequantisation and the MFMAs of a SIMD's two waves still overlap only in part (2.1 us a round of
-// 128 k with the chip full, 1.0 PFLOP/s; of 75 us for the case below 20 less without the arithmetic and 18 less with one
-// MFMA instead of all).  gate|up 28672 x 4096 of Q4_K with its activation: 256 rows 78 (gemm_bs.hip) -> 74 us, 128 rows
-// 68 (gemm_q32.hip) -> 54, 701 rows 229 (copy, library, activation) -> 208; 4096 x 14336 at 400 rows 115 (copy,
-// library) -> 84, 4096 x 4096 42 -> 37.  Plain products of up to 256 rows with few columns stay with the kernels
-// above: the autotuner times them all.
+// What bounds it: vector issue and MFMAs need about 1000 of the SIMD's cycles a step of 64 k each (6.5 vector
+// instructions an MFMA) and would overlap; a step takes 1900 (45 % MFMA, 55 % vector pipe busy), the rest is lost where
+// the two waves of a SIMD wait for each other at the barrier.  Kept out of the way of the MFMAs: waits for LDS (operands
+// are pinned behind the previous half-step; without that the compiler waits for every outstanding read: 78 -> 75 us),
+// the DMA's issue (one instruction after an MFMA, not all behind the barrier: -> 71 us), address arithmetic (scalar).
+// gate|up 28672 x 4096 of Q4_K with its activation: 256 rows 78 (gemm_bs.hip) -> 71 us, 128 rows 68 (gemm_q32.hip) ->
+// 52, 701 rows 229 (copy, library, activation) -> 200; 4096 x 14336 at 400 rows 115 (copy, library) -> 80, 4096 x 4096
+// 42 -> 36.  Plain products of up to 256 rows with few columns stay with the other kernels: the autotuner times them.
+#include <type_traits>
+
 #include "qstage.h"
 
 namespace la {
 
 typedef float f32x16w __attribute__((ext_vector_type(16)));
 
-// Raw bytes and scales of one lane's weight row (column c of a block of 32) for a step: row `c & 15` of one of the
-// block's two 16-row tiles.  p: which half of the tile's 128 k, gs: which 32 of the step's 64 k.
+// LDS addresses of a lane's weight row (column c of a block of 32: row c & 15 of one of the block's two 16-row tiles)
+// that no step changes; a step adds scalars and flips bits, one instruction each.
+struct WdLane {
+  uint32_t raw, raw2, q, d;
+};
+// keeps the loads of v before this place: without it the compiler waits for every outstanding LDS read at v's first use
+template <typename T>
+LA_DEV void wd_pin(T& v) {
+  asm volatile("" : "+v"(v));
+}
+
+// Raw bytes and scales for a step.  P: which half of the tile's 128 k, gs: which 32 of the step's 64 k.  load(): wo, qo
+// the offsets of the macro's slot and of the quad's buffer, j the step, o / oq of the column block's tile.
 template <int FMT> struct WdW;
 
 template <> struct WdW<FMT_Q4_K> {
@@ -48,12 +63,17 @@ template <> struct WdW<FMT_Q4_K> {
   u32x4 q;
   uint32_t scm, dd;
   float D, Mn;
-  LA_DEV void load(const uint8_t* l, const uint8_t* qd, int t, int gs, int r, int h, int) {
-    const int i = (t >> 2) & 3;
-    q = *(const u32x4*)(l + 64 * r + 16 * ((2 * (t & 1) + h) ^ (r >> 2)));
-    scm = *(const uint32_t*)(qd + sk_quad(r, i) + 4 * (t & 3));
-    dd = *(const uint32_t*)(qd + 1024 + 16 * r + 4 * i);
+  LA_DEV static WdLane lane(uint32_t raw, uint32_t qd, int r, int h, int gs, int) {
+    return WdLane{raw + 64 * r + 16 * (h ^ (r >> 2)), 0, qd + sk_quad(r, 0), qd + 1024 + 16 * r};
   }
+  template <int P>
+  LA_DEV void load(const uint8_t* lds, const WdLane& a, uint32_t wo, uint32_t qo, int t, int o, int oq) {
+    const int i = (t >> 2) & 3;
+    q = *(const u32x4*)(lds + ((a.raw ^ (32 * P)) + wo) + o);
+    scm = *(const uint32_t*)(lds + ((a.q ^ (16 * i)) + (qo + 4 * (t & 3))) + oq);
+    dd = *(const uint32_t*)(lds + (a.d + (qo + 4 * i)) + oq);
+  }
+  LA_DEV void pin() { wd_pin(q), wd_pin(scm), wd_pin(dd); }
   LA_DEV void prep(int gs) {
     const uint32_t s = scm >> (16 * gs);
     D = h2f(dd & 0xFFFFu) * 512.f * ubyte_f(s, 0);
@@ -90,15 +110,22 @@ template <> struct WdW<FMT_Q6_K> {
   }
   u32x4 l4, h4;
   int sc;
-  uint16_t dbits;
+  uint32_t dbits;
   float D;
-  LA_DEV void load(const uint8_t* l, const uint8_t* qd, int t, int gs, int r, int h, int idx) {
-    const int i = (t >> 2) & 3, e = idx + (t >> 2);
-    l4 = *(const u32x4*)(l + 64 * r + 16 * ((2 * gs + h) ^ (r >> 2)));
-    h4 = *(const u32x4*)(l + 1024 + 32 * r + 16 * (h ^ (r >> 3)));
-    sc = *(const int8_t*)(qd + sk_quad(r, i) + 8 * ((t >> 1) & 1) + 4 * (t & 1) + 2 * gs + h);
-    dbits = *(const uint16_t*)(qd + 1024 + 16 * r + 4 * ((e >> 1) - ((e - i) >> 1)) + 2 * (e & 1));
+  // the quad's first d is at the lane's parity in its aligned dwords (4 super-blocks: an even number)
+  LA_DEV static WdLane lane(uint32_t raw, uint32_t qd, int r, int h, int gs, int idx) {
+    return WdLane{raw + 64 * r + 16 * ((2 * gs + h) ^ (r >> 2)), raw + 1024 + 32 * r + 16 * (h ^ (r >> 3)),
+                  qd + sk_quad(r, 0) + 2 * gs + h, qd + 1024 + 16 * r + 2 * (idx & 1)};
   }
+  template <int P>
+  LA_DEV void load(const uint8_t* lds, const WdLane& a, uint32_t wo, uint32_t qo, int t, int o, int oq) {
+    const int i = (t >> 2) & 3;
+    l4 = *(const u32x4*)(lds + (a.raw + wo) + o);
+    h4 = *(const u32x4*)(lds + (a.raw2 + wo) + o);
+    sc = *(const int8_t*)(lds + ((a.q ^ (16 * i)) + (qo + 4 * (t & 3))) + oq);
+    dbits = *(const uint16_t*)(lds + (a.d + (qo + 2 * i)) + oq);
+  }
+  LA_DEV void pin() { wd_pin(l4), wd_pin(h4), wd_pin(sc), wd_pin(dbits); }
   LA_DEV void prep(int) { D = h2f(dbits) * (float)sc; }
   template <int S>
   LA_DEV bf16x8 deq(int t, int gs) const {
@@ -126,12 +153,17 @@ template <> struct WdW<FMT_Q8_0> {
     sk_dma16(p.b + 128 * m, dst + 1024);
   }
   u32x4 q;
-  uint16_t dbits;
+  uint32_t dbits;
   float D;
-  LA_DEV void load(const uint8_t* l, const uint8_t* qd, int t, int gs, int r, int h, int) {
-    q = *(const u32x4*)(l + 128 * r + 16 * ((4 * (t & 1) + 2 * gs + h) ^ (r >> 1)));
-    dbits = *(const uint16_t*)(qd + sk_quad(r, (t >> 2) & 3) + 4 * (t & 3) + 2 * gs);
+  LA_DEV static WdLane lane(uint32_t raw, uint32_t qd, int r, int h, int gs, int) {
+    return WdLane{raw + 128 * r + 16 * ((2 * gs + h) ^ (r >> 1)), 0, qd + sk_quad(r, 0) + 2 * gs, 0};
   }
+  template <int P>
+  LA_DEV void load(const uint8_t* lds, const WdLane& a, uint32_t wo, uint32_t qo, int t, int o, int oq) {
+    q = *(const u32x4*)(lds + ((a.raw ^ (64 * P)) + wo) + o);
+    dbits = *(const uint16_t*)(lds + ((a.q ^ (16 * ((t >> 2) & 3))) + (qo + 4 * (t & 3))) + oq);
+  }
+  LA_DEV void pin() { wd_pin(q), wd_pin(dbits); }
   LA_DEV void prep(int) { D = h2f(dbits); }
   template <int S>
   LA_DEV bf16x8 deq(int, int) const {
@@ -168,11 +200,11 @@ LA_DEV void wd_tile(uint8_t* lds, const QW& w, int tile, int m0, const bf16* __r
   const int t0 = 2 * M0, t1 = 2 * mend;
 
   // sources: the wave fetches RB pieces (8 rows) of X and one of the 8 weight tiles (GLU: 0-3 gate, 4-7 up)
-  const bf16* xp[RB];
+  uint32_t xo[RB];   // bytes; a scalar base and a 32-bit offset need no address arithmetic in the vector pipe
 #pragma unroll
   for (int i = 0; i < RB; ++i) {
     const int row = 8 * (wave * RB + i) + (lane >> 3);
-    xp[i] = X + (size_t)min(m0 + row, M - 1) * ldx + ((lane & 7) ^ ((row >> 1) & 7)) * 8;
+    xo[i] = ((uint32_t)min(m0 + row, M - 1) * ldx + ((lane & 7) ^ ((row >> 1) & 7)) * 8) * 2;
   }
   const bool up = GLU && wave >= 4;
   auto trow = [&](int tl, int i) {   // weight row of row i of tile tl (rows past N repeat the last)
@@ -184,21 +216,19 @@ LA_DEV void wd_tile(uint8_t* lds, const QW& w, int tile, int m0, const bf16* __r
   uint8_t* quads = wring + C::WB;
   auto issue_x = [&](int t, int slot) {
 #pragma unroll
-    for (int i = 0; i < RB; ++i) sk_dma16(xp[i] + min(t, t1 - 1) * 64, lds + slot * C::XB + (wave * RB + i) * 1024);
+    for (int i = 0; i < RB; ++i) sk_dma16((const uint8_t*)(X + min(t, t1 - 1) * 64) + xo[i], lds + slot * C::XB + (wave * RB + i) * 1024);
   };
   auto issue_w = [&](int m, int slot) { W::issue(wp, min(m, mend - 1), wring + slot * C::WS + wave * W::BYTES); };
   auto issue_quad = [&](int qd) { SkW<FMT>::issue_quad(wp.q, 4 * qd, quads + ((qd & 1) * 8 + wave) * W::QBYTES, lane); };
-  // the wave's column block b: tiles tb(b) and tb(b) + 1; the lane's column is row r & 15 of tile tb(b) + (r >> 4)
-  auto tb = [&](int b) { return GLU ? 4 * b + 2 * nw : 4 * nw + 2 * b; };
-  int idx[2];
-#pragma unroll
-  for (int b = 0; b < 2; ++b) idx[b] = trow(tb(b) + (r >> 4), r & 15) * (w.K >> 8);
-  auto fetch = [&](W (&f)[2], int t, int wslot) {
-#pragma unroll
-    for (int b = 0; b < 2; ++b) {
-      const int tl = tb(b) + (r >> 4);
-      f[b].load(wring + wslot * C::WS + tl * W::BYTES, quads + (((t >> 4) & 1) * 8 + tl) * W::QBYTES, t, gs, r & 15, h, idx[b]);
-    }
+  // the wave's column block b: tiles tl(b) and tl(b) + 1; the lane's column is row r & 15 of tile tl(b) + (r >> 4)
+  constexpr int TB = GLU ? 4 : 2;    // tiles from block 0 to block 1
+  const int tl0 = (GLU ? 2 : 4) * nw + (r >> 4);
+  const WdLane la0 = W::lane(C::XS + tl0 * W::BYTES, C::XS + C::WB + tl0 * W::QBYTES, r & 15, h, gs, trow(tl0, r & 15) * (w.K >> 8));
+  const WdLane la1 = W::lane(C::XS + tl0 * W::BYTES, C::XS + C::WB + tl0 * W::QBYTES, r & 15, h, gs, trow(tl0 + TB, r & 15) * (w.K >> 8));
+  auto fetch = [&](W (&f)[2], int t, auto odd, int wslot) {
+    const uint32_t wo = wslot * C::WS, qo = ((t >> 4) & 1) * 8 * W::QBYTES;
+    f[0].template load<decltype(odd)::value>(lds, la0, wo, qo, t, 0, 0);
+    f[1].template load<decltype(odd)::value>(lds, la1, wo, qo, t, TB * W::BYTES, TB * W::QBYTES);
   };
 
   f32x16w acc[RB][2];
@@ -222,60 +252,67 @@ LA_DEV void wd_tile(uint8_t* lds, const QW& w, int tile, int m0, const bf16* __r
   issue_x(t0 + 1, 1);
   asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(2 * RB + W::PIECES) : "memory");
   W f[2][2];
-  fetch(f[0], t0, 0);
+  fetch(f[0], t0, std::false_type{}, 0);
   int xs = 0, ws = 0;                // slots of step t's X and of its macro
   // Half a step (one MFMA per block pair and 16 k) is multiplied while the next half is dequantised: the second half
   // of step t - 1 beside the first dequantisation of step t, so a wave has vector work between all its MFMAs.
-  bf16x8 a0[RB], a1[RB], b0[2], b1[2];
+  u32x4 a0[RB], a1[RB];
+  bf16x8 b0[2], b1[2];
 #pragma unroll
-  for (int i = 0; i < RB; ++i) a1[i] = bf16x8{};
+  for (int i = 0; i < RB; ++i) a1[i] = u32x4{};
 #pragma unroll
   for (int b = 0; b < 2; ++b) b1[b] = bf16x8{};
-  auto mul = [&](const bf16x8 (&a)[RB], const bf16x8 (&bb)[2]) {
+  auto mul = [&](const u32x4 (&a)[RB], const bf16x8 (&bb)[2]) {
 #pragma unroll
     for (int i = 0; i < RB; ++i)
 #pragma unroll
-      for (int b = 0; b < 2; ++b) acc[i][b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[i], bb[b], acc[i][b], 0, 0, 0);
+      for (int b = 0; b < 2; ++b) acc[i][b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a[i]), bb[b], acc[i][b], 0, 0, 0);
   };
-  auto mix = [&]() {                 // an MFMA, then its share of the vector instructions
+  auto mix = [&](bool dma) {         // an MFMA, then its share of the vector instructions and of the DMA
 #pragma unroll
     for (int i = 0; i < 2 * RB; ++i) {
       __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
       __builtin_amdgcn_sched_group_barrier(0x002, 6, 0);
+      if (dma) __builtin_amdgcn_sched_group_barrier(0x010, 1, 0);
     }
   };
-  auto step = [&](W (&cur)[2], W (&nxt)[2], int t, bool odd) {
+  auto step = [&](W (&cur)[2], W (&nxt)[2], int t, auto odd) {
+#pragma unroll
+    for (int i = 0; i < RB; ++i) wd_pin(a1[i]);
+    cur[0].pin(), cur[1].pin();
     asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(RB + W::PIECES) : "memory");
     if ((t & 15) == 0 && t != t0) issue_quad((t >> 4) + 1);
-    issue_x(t + 2, xs == 0 ? 2 : xs - 1);
-    if (!odd) issue_w((t >> 1) + 2, ws == 0 ? 2 : ws - 1);
     const uint8_t* x = lds + xs * C::XB;
 #pragma unroll
-    for (int i = 0; i < RB; ++i) a0[i] = *(const bf16x8*)(x + aoff[0] + i * (32 * 128));
+    for (int i = 0; i < RB; ++i) a0[i] = *(const u32x4*)(x + aoff[0] + i * (32 * 128));
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int b = 0; b < 2; ++b) {
       cur[b].prep(gs);
       b0[b] = cur[b].template deq<0>(t, gs);
     }
+    issue_x(t + 2, xs == 0 ? 2 : xs - 1);
+    if (!decltype(odd)::value) issue_w((t >> 1) + 2, ws == 0 ? 2 : ws - 1);
     mul(a1, b1);
-    mix();
+    mix(true);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int i = 0; i < RB; ++i) a1[i] = *(const bf16x8*)(x + aoff[1] + i * (32 * 128));
-    if (odd) ws = ws == 2 ? 0 : ws + 1;
-    fetch(nxt, t + 1, ws);
+    for (int i = 0; i < RB; ++i) wd_pin(a0[i]);
+#pragma unroll
+    for (int i = 0; i < RB; ++i) a1[i] = *(const u32x4*)(x + aoff[1] + i * (32 * 128));
+    if (decltype(odd)::value) ws = ws == 2 ? 0 : ws + 1;
+    fetch(nxt, t + 1, std::bool_constant<!decltype(odd)::value>{}, ws);
     xs = xs == 2 ? 0 : xs + 1;
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int b = 0; b < 2; ++b) b1[b] = cur[b].template deq<1>(t, gs);
     mul(a0, b0);
-    mix();
+    mix(false);
     __builtin_amdgcn_sched_barrier(0);
   };
   for (int t = t0; t < t1; t += 2) {
-    step(f[0], f[1], t, false);
-    step(f[1], f[0], t + 1, true);
+    step(f[0], f[1], t, std::false_type{});
+    step(f[1], f[0], t + 1, std::true_type{});
   }
   mul(a1, b1);
   asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");   // every DMA has landed, every read is done
@@ -365,7 +402,7 @@ extern "C" int la_wgemm(int fmt, const void* const* a, int N, int K, const void*
                         int ldo, long slab, int out_bf16, int rb, void* stream) {
   using namespace la;
   const int total = K >> 7, per = splits > 0 ? (total + splits - 1) / splits : 0;
-  if (M < 1 || N < 1 || (K & 255) || splits < 1 || (long)per * (splits - 1) >= total || ldo < N || ldx < K || (ldx & 7) ||
+  if (M < 1 || N < 1 || (K & 255) || splits < 1 || (long)per * (splits - 1) >= total || ldo < N || ldx < K || (ldx & 7) || (long)M * ldx >= (1L << 31) ||
       (out_bf16 ? splits != 1 : slab < (long)M * ldo) || wd_odd(fmt, N, K))
     return -1;
   const QW w = wd_qw(a, N, K);
@@ -395,7 +432,7 @@ extern "C" int la_wgemm2(const void* const* a, int Na, const void* const* b, int
   using namespace la;
   const int total = K >> 7, per = splits > 0 ? (total + splits - 1) / splits : 0;
   if (M < 1 || Na < 1 || Nb < 1 || (K & 255) || splits < 1 || (long)per * (splits - 1) >= total || ldo < Na + Nb || ldx < K ||
-      (ldx & 7) || (out_bf16 ? splits != 1 : slab < (long)M * ldo) || wd_odd(FMT_Q6_K, Nb, K))
+      (ldx & 7) || (long)M * ldx >= (1L << 31) || (out_bf16 ? splits != 1 : slab < (long)M * ldo) || wd_odd(FMT_Q6_K, Nb, K))
     return -1;
   const QW wa = wd_qw(a, Na, K), wb = wd_qw(b, Nb, K);
   const int ta = (Na + 127) / 128;
@@ -415,7 +452,7 @@ extern "C" int la_wgemm2(const void* const* a, int Na, const void* const* b, int
 extern "C" int la_wgemm_glu(int fmt, const void* const* a, int oa, const void* const* b, int ob, int F, int K, const void* X,
                             int ldx, int M, void* out, int ldo, int act, int rb, void* stream) {
   using namespace la;
-  if (M < 1 || F < 1 || (K & 255) || ldo < F || ldx < K || (ldx & 7) || (act != 0 && act != 3) || wd_odd(fmt, oa + F, K) ||
+  if (M < 1 || F < 1 || (K & 255) || ldo < F || ldx < K || (ldx & 7) || (long)M * ldx >= (1L << 31) || (act != 0 && act != 3) || wd_odd(fmt, oa + F, K) ||
       wd_odd(fmt, ob + F, K))
     return -1;
   const QW w = wd_qw(a, oa + F, K);
