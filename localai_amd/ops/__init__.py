@@ -837,6 +837,7 @@ GQ_TILES = {0: (256, 256), 1: (256, 128), 2: (128, 256), 3: (128, 128), 4: (256,
             7: (128, 256), 8: (256, 128), 12: (128, 128), 14: (64, 256),
             # software-pipelined schedules of 0, 1, 3, 6, 7
             10: (256, 256), 11: (256, 128), 13: (128, 128), 16: (256, 256), 17: (128, 256)}
+WIDE_TILES = {22: (128, 128), 24: (256, 128)}   # gemm_wide.hip (20 + rows / 64): the raw scale planes, no la_gemm_scales
 # LOCALAI_AMD_TILE_GEMM=0 restores the round-2 path (hipBLASLt on bf16 weight copies)
 TILE_GEMM = os.environ.get("LOCALAI_AMD_TILE_GEMM", "1") == "1"
 # M > MID_MAX_M (prefill chunks): "blas" = dequantise into a scratch buffer + library GEMM, "tile" =
@@ -858,6 +859,9 @@ _TILE2_TILES = (7, 8, 12)
 def _run_tile(x, ws, S, out, Ntot, tile):
     """out: fp32 slabs [S, M, Ntot], or a bf16 [M, Ntot] matrix (S == 1).  Two weights of a
     Q4_K/Q6_K mix (q|k + v) run as ONE launch (la_qgemm_tile2)."""
+    if tile in WIDE_TILES:
+        _run_w(x, ws, S, out, Ntot, tile - 20)
+        return
     M, K = x.shape
     bf = out.dtype == torch.bfloat16
     esz = 2 if bf else 4
@@ -973,10 +977,6 @@ def w_ok(ws: Sequence[QWeight]) -> bool:
     return _has("la_wgemm") and all(w.fmt in W_FMTS and w.planes[0] is not None and _skinny_ok(w) for w in ws)
 
 
-def _w_grid(M: int, N: int, rb: int) -> int:
-    return -(-M // (64 * rb)) * -(-N // 128)
-
-
 def _w_split_ok(K: int, S: int) -> bool:
     return S >= 1 and -(-(K // 128) // S) * (S - 1) < K // 128
 
@@ -1014,7 +1014,7 @@ def _q32_grid(M: int, N: int, var: int) -> int:
 
 
 def _tile_grid(M: int, N: int, tile: int) -> int:
-    bm, bn = GQ_TILES[tile]
+    bm, bn = GQ_TILES.get(tile) or WIDE_TILES[tile]
     return -(-M // bm) * -(-N // bn)
 
 
@@ -1067,11 +1067,11 @@ def _autotune_mid(x, ws, key, Ntot):
                 if S <= min(8, K // 256) and _tile_split_ok(K, S):
                     cands.append(("bs", S, v))
     if w_ok(ws):
-        for rb in (4, 2) if M > 128 else (2,):
-            base = max(1, round(256 / _w_grid(M, Ntot, rb)))
+        for t in (24, 22) if M > 128 else (22,):
+            base = max(1, round(256 / _tile_grid(M, Ntot, t)))
             for S in sorted({1, max(1, base // 2), base, base * 2}):
                 if S <= min(8, K // 256) and _w_split_ok(K, S):
-                    cands.append(("w", S, rb))
+                    cands.append(("tile", S, t))
     if not cands or not TILE_GEMM:
         cands = [("blas", 0, 0)]
     outs = {S: torch.empty(S, M, Ntot, dtype=torch.float32, device=x.device) for _, S, _ in cands if S > 1}
@@ -1084,8 +1084,6 @@ def _autotune_mid(x, ws, key, Ntot):
             fn = lambda S=S, t=t: _run_tile(x, ws, S, outs[S], Ntot, t)  # noqa: E731
         elif kind == "bs":
             fn = lambda S=S, t=t: _run_bs(x, ws, S, outs[S], Ntot, t)  # noqa: E731
-        elif kind == "w":
-            fn = lambda S=S, t=t: _run_w(x, ws, S, outs[S], Ntot, t)  # noqa: E731
         else:
             fn = lambda S=S, t=t: _run_q32(x, ws, S, outs[S], Ntot, t)  # noqa: E731
         fn()
@@ -1109,13 +1107,13 @@ def _autotune_mid(x, ws, key, Ntot):
 
 
 # Time of one K step of a workgroup (us; a step is 64 k of a 256 x 256 tile, 128 k of a 256 x 128 one), chip full
-_STEP_US = {"tile": {FMT_Q4_K: 1.75, FMT_Q6_K: 2.05, FMT_Q8_0: 1.85}, "w": {FMT_Q4_K: 2.1, FMT_Q6_K: 2.4, FMT_Q8_0: 2.2}}
+_STEP_US = {6: {FMT_Q4_K: 1.75, FMT_Q6_K: 2.05, FMT_Q8_0: 1.85}, 24: {FMT_Q4_K: 2.1, FMT_Q6_K: 2.4, FMT_Q8_0: 2.2}}
 QUANT_MAX_M = 1280
 
 
 @functools.lru_cache(maxsize=4096)
 def _quant_plan(M: int, K: int, ws: Tuple[Tuple[int, int], ...], glu: bool, tile_ok: bool, wide_ok: bool) -> Optional[tuple]:
-    """(kind, S, tile) of the product that reads the quantised weights ((fmt, N), ...) itself, or None where a bf16 copy
+    """(S, tile) of the product that reads the quantised weights ((fmt, N), ...) itself, or None where a bf16 copy
     and the library's GEMM are faster: the rule for MID_MAX_M < M <= QUANT_MAX_M rows.  A rule and no autotuning, since
     the length of a prompt chunk differs per call.
 
@@ -1133,17 +1131,17 @@ def _quant_plan(M: int, K: int, ws: Tuple[Tuple[int, int], ...], glu: bool, tile
     if glu:
         lib_us += 3 + M * N * 3 / 4e6                    # the activation's own pass
     best, best_us = None, 0.95 * lib_us
-    for kind, bn, bk, ok in (("tile", 256, 64, tile_ok), ("w", 128, 128, wide_ok)):
+    for tile, bn, bk, ok in ((6, 256, 64, tile_ok), (24, 128, 128, wide_ok)):
         if not ok:
             continue
-        step = max(_STEP_US[kind][f] for f, _ in ws) + (0.15 if glu and kind == "tile" else 0)
+        step = max(_STEP_US[tile][f] for f, _ in ws) + (0.15 if glu and tile == 6 else 0)
         tiles = -(-M // 256) * sum(-(-n // bn) for _, n in ws)
         for S in range(1, 2 if glu else 9):
-            if not (_tile_split_ok(K, S) if kind == "tile" else _w_split_ok(K, S)):
+            if not (_tile_split_ok(K, S) if tile == 6 else _w_split_ok(K, S)):
                 continue
             us = -(-tiles * S // 256) * -(-(K // bk) // S) * step + 8 + (S * M * N * 8 / 4.5e6 if S > 1 else 0)
             if us < best_us:
-                best, best_us = (kind, S, 6 if kind == "tile" else 4), us
+                best, best_us = (S, tile), us
     return best
 
 
@@ -1158,7 +1156,7 @@ def _plan_quant(M: int, K: int, ws: Sequence[QWeight], glu: bool = False) -> Opt
     tile_ok = len(ws) == 1 and _has("la_qgemm_tile")
     key = (M, K, tuple((w.fmt, w.N) for w in ws), glu)
     plan = _quant_plan(*key, tile_ok, w_ok(ws))
-    if plan is not None and plan[0] == "tile" and w.gsc is None:
+    if plan is not None and plan[1] == 6 and w.gsc is None:
         if torch.cuda.is_current_stream_capturing() or torch.cuda.mem_get_info(w.device)[0] < (4 << 30) + w.N * w.K // 8:
             plan = _quant_plan(*key, False, w_ok(ws))
     return plan
@@ -1200,7 +1198,7 @@ def linear_multi(x: torch.Tensor, ws: Sequence[QWeight], bias: Optional[torch.Te
     use_skinny = (M <= SKINNY_MAX_M and skinny_ok) if force is None else force == "skinny"
     tile_ok = TILE_GEMM and all(w.tile_ok for w in ws) and (_has("la_qgemm_tile") or _has("la_qgemm32") or _has("la_bsgemm"))
     S, tile, kind = 0, 0, None
-    if force is not None and force.split(":")[0] in ("q32", "bs", "w"):
+    if force is not None and force.split(":")[0] in ("q32", "bs"):
         kind, v, s_ = force.split(":")
         tile, S = int(v), int(s_)
     elif force is not None and force.startswith("tile"):
@@ -1218,7 +1216,7 @@ def linear_multi(x: torch.Tensor, ws: Sequence[QWeight], bias: Optional[torch.Te
         if choice is None and tile_ok and _has("la_qgemm_tile"):
             t, s_ = pick_tile(M, [w.N for w in ws], K)
             choice = ("tile", s_, t)
-        if choice is not None and choice[0] in ("tile", "q32", "bs", "w"):
+        if choice is not None and choice[0] in ("tile", "q32", "bs"):
             kind, S, tile = choice
     elif force is None and not use_skinny and tile_ok and PREFILL_GEMM == "tile":
         tile, S = pick_tile(M, [w.N for w in ws], K)   # prefill: heuristic, never tuned inline
@@ -1226,10 +1224,10 @@ def linear_multi(x: torch.Tensor, ws: Sequence[QWeight], bias: Optional[torch.Te
     elif force is None and not use_skinny:
         plan = _plan_quant(M, K, ws)
         if plan is not None:
-            kind, S, tile = plan
-    if kind in ("tile", "q32", "bs", "w") and S == 1 and out_slabs is None:
+            kind, (S, tile) = "tile", plan
+    if kind in ("tile", "q32", "bs") and S == 1 and out_slabs is None:
         y = torch.empty(M, Ntot, dtype=torch.bfloat16, device=x.device)
-        {"tile": _run_tile, "q32": _run_q32, "bs": _run_bs, "w": _run_w}[kind](x, ws, 1, y, Ntot, tile)
+        {"tile": _run_tile, "q32": _run_q32, "bs": _run_bs}[kind](x, ws, 1, y, Ntot, tile)
         return Partial(y, bias)
     if S:
         out = out_slabs
@@ -1239,8 +1237,6 @@ def linear_multi(x: torch.Tensor, ws: Sequence[QWeight], bias: Optional[torch.Te
             _run_tile(x, ws, S, out, Ntot, tile)
         elif kind == "bs":
             _run_bs(x, ws, S, out, Ntot, tile)
-        elif kind == "w":
-            _run_w(x, ws, S, out, Ntot, tile)
         else:
             _run_q32(x, ws, S, out, Ntot, tile)
         return Partial(out, bias)
@@ -1295,12 +1291,11 @@ def _glu_pair(ws: Sequence[QWeight], F: int):
 
 
 def _run_glu(x: torch.Tensor, pair, F: int, mode: int, tile: int, out: torch.Tensor) -> None:
-    """tile < 100: gemm_q.hip tile id; 100 + v: gemm_q32.hip variant v; 200 + v: gemm_bs.hip variant v; 300 + rb:
-    gemm_wide.hip."""
+    """tile < 100: GQ_TILES or WIDE_TILES id; 100 + v: gemm_q32.hip variant v; 200 + v: gemm_bs.hip variant v."""
     M, K = x.shape
     wa, oa, wb, ob = pair
-    if tile >= 300:
-        _run_w_glu(x, pair, F, mode, tile - 300, out)
+    if tile in WIDE_TILES:
+        _run_w_glu(x, pair, F, mode, tile - 20, out)
         return
     if tile >= 200:
         _run_bs_glu(x, pair, F, mode, tile - 200, out)
@@ -1359,7 +1354,7 @@ def glu_linear(x: torch.Tensor, ws: Sequence[QWeight], F: int, mode: int,
         if x.dtype != torch.bfloat16 or not x.is_contiguous() or K != ws[0].K:
             raise ValueError("glu_linear: x must be contiguous bf16 [M, K]")
         out = torch.empty(M, F, dtype=torch.bfloat16, device=x.device)
-        _run_glu(x, _glu_pair(ws, F), F, mode, plan[2] if plan[0] == "tile" else 300 + plan[2], out)
+        _run_glu(x, _glu_pair(ws, F), F, mode, plan[1], out)
         return out
     pair = _glu_pair(ws, F)
     if pair is None:
@@ -1377,15 +1372,12 @@ def glu_linear(x: torch.Tensor, ws: Sequence[QWeight], F: int, mode: int,
         out = torch.empty(M, F, dtype=torch.bfloat16, device=x.device)
         t_ref = _time_cold(lambda: act(linear_multi(x, ws), F, mode))
         best, best_t = None, t_ref
-        cands = [6, 7, 8] if M > 128 else [7, 12, 14]
-        if q32_ok([pair[0]], 9) and pair[0].fmt == pair[2].fmt:
-            # (128-row tiles at M > 128 -- 107 / 105, two row tiles to fill the chip -- were timed
-            # and never won: r5_glu_bench.log)
-            cands += [109, 108, 104] if M > 128 else [109, 108, 107]
-        if bs_ok([pair[0], pair[2]]) and pair[0].fmt == pair[2].fmt and F % 4 == 0:
-            cands += [200, 203] if M > 128 else [201]
         if w_ok([pair[0], pair[2]]) and pair[0].fmt == pair[2].fmt:
-            cands += [304, 302] if M > 128 else [302]
+            # the others lose at every size (28672 x 4096, Q4_K: 256 rows 73 us against 84 to 95, 128 rows 55 against 67 to
+            # 75), but one timed call now and then says otherwise
+            cands = [24, 22] if M > 128 else [22]
+        else:
+            cands = [6, 7, 8] if M > 128 else [7, 12, 14]
         for t in cands:
             tt = _time_cold(lambda t=t: _run_glu(x, pair, F, mode, t, out))
             if tt < best_t:

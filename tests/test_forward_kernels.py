@@ -145,9 +145,9 @@ def test_wide_products(t, N, K, S, M, rb):
     ref = x.float() @ w.ref.t()
     bound = 2 ** -9 * (x.float().abs() @ w.ref.abs().t()) + 1e-5
     slabs = torch.empty(S, M, N, device=DEV)
-    y = ops.linear(x.to(DEV), w, force=f"w:{rb}:{S}", out_slabs=slabs).dense().cpu()
+    y = ops.linear(x.to(DEV), w, force=f"tile:{20 + rb}:{S}", out_slabs=slabs).dense().cpu()
     assert ((y - ref).abs() <= bound).all()
-    y = ops.linear(x.to(DEV), w, force=f"w:{rb}:1").dense().cpu()
+    y = ops.linear(x.to(DEV), w, force=f"tile:{20 + rb}:1").dense().cpu()
     assert ((y - ref).abs() <= bound + 2 ** -8 * ref.abs()).all()
 
 
@@ -163,7 +163,7 @@ def test_wide_gated(t, F, K, M, rb):
     bound = 1.2 * eg * (u.abs() + eu) + s.abs() * eu + 2 ** -8 * (s * u).abs() + 1e-5
     for pair in ((a, 0, b, 0), (ops.concat_rows([a, b]), 0, ops.concat_rows([a, b]), F)):
         h = torch.empty(M, F, dtype=torch.bfloat16, device=DEV)
-        ops._run_glu(x.to(DEV), pair, F, ops.ACT_SWIGLU, 300 + rb, h)
+        ops._run_glu(x.to(DEV), pair, F, ops.ACT_SWIGLU, 20 + rb, h)
         assert ((h.float().cpu() - s * u).abs() <= bound).all()
 
 
@@ -172,20 +172,20 @@ def test_wide_pair(M, rb, S):
     """Q4_K and Q6_K side by side against each alone."""
     ws = [_weight(200, 1536, GGMLType.Q4_K, 1), _weight(72, 1536, GGMLType.Q6_K, 2)]
     x = torch.randn(M, 1536, generator=torch.Generator().manual_seed(M)).to(torch.bfloat16).to(DEV)
-    y = ops.linear_multi(x, ws, force=f"w:{rb}:{S}", out_slabs=torch.empty(S, M, 272, device=DEV))
-    alone = [ops.linear(x, w, force=f"w:{rb}:{S}", out_slabs=torch.empty(S, M, w.N, device=DEV)) for w in ws]
+    y = ops.linear_multi(x, ws, force=f"tile:{20 + rb}:{S}", out_slabs=torch.empty(S, M, 272, device=DEV))
+    alone = [ops.linear(x, w, force=f"tile:{20 + rb}:{S}", out_slabs=torch.empty(S, M, w.N, device=DEV)) for w in ws]
     assert torch.equal(y.t, torch.cat([p.t for p in alone], -1))
 
 
-@pytest.mark.parametrize("t,N,K,M,kind", [(GGMLType.Q4_K, 2048, 8192, 257, "w"), (GGMLType.Q4_K, 2050, 8192, 512, "w"), (GGMLType.Q6_K, 4096, 14336, 701, "tile"),
-                                          (GGMLType.Q8_0, 4096, 14336, 1024, "tile"), (GGMLType.Q4_K, 4096, 4096, 1280, None)])
-def test_prompt_plan(t, N, K, M, kind):
+@pytest.mark.parametrize("t,N,K,M,tile", [(GGMLType.Q4_K, 2048, 8192, 257, 24), (GGMLType.Q4_K, 2050, 8192, 512, 24), (GGMLType.Q6_K, 4096, 14336, 701, 6),
+                                          (GGMLType.Q8_0, 4096, 14336, 1024, 6), (GGMLType.Q4_K, 4096, 4096, 1280, None)])
+def test_prompt_plan(t, N, K, M, tile):
     """Either side of the line between the quantised products and the copy with the library's: same sums, and the gated
     form through its entry.  Every path rounds a weight to bf16 and sums in fp32; the copy's result is rounded once more."""
     w = _weight(N, K, t, N + K)
     x = torch.randn(M, K, generator=torch.Generator().manual_seed(M)).to(torch.bfloat16).to(DEV)
     plan = ops._plan_quant(M, K, [w])
-    assert (plan[0] if plan else None) == kind
+    assert (plan[1] if plan else None) == tile
     wf = w.ref.to(DEV)
     ref, bound = x.float() @ wf.t(), 2 ** -9 * (x.float().abs() @ wf.abs().t()) + 1e-4
     assert ((ops.linear(x, w).dense() - ref).abs() <= bound + 2 ** -8 * ref.abs()).all()
