@@ -3850,8 +3850,7 @@ def _moe32_var(env: int, T: int, fmt: int = FMT_Q4_K, down: bool = False) -> int
     # var 17 (64-row chunks) 167 + 82 / 172 + 86 vs var 9's 166 + 91 / var 4's 180 + 91; below
     # MOE32_SMALL_T var 9 (32-row tiles, 4 workgroups per CU) stays for the smallest batches
     if T >= MOE32_LIVE_BIG_T:
-        # var 19's 64-column waves spill with Q6_K / Q8_0 fragments (the launcher maps them to 15)
-        return 19 if fmt == FMT_Q4_K else 15
+        return 19
     return 9 if T < MOE32_SMALL_T else 17
 
 

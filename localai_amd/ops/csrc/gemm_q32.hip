@@ -39,6 +39,12 @@ LA_DEV void q32_glds4(const void* g, void* l) {
   __builtin_amdgcn_global_load_lds(g, (__attribute__((address_space(3))) void*)l, 4, 0, 0);
 }
 
+// Keeps a load of v before this place: without it the compiler waits for every outstanding LDS read at v's first use.
+template <typename T>
+LA_DEV void q32_pin(T& v) {
+  asm volatile("" : "+v"(v));
+}
+
 template <int N>
 LA_DEV void q32_vmwait() {
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
@@ -90,38 +96,36 @@ template <> struct Q32F<FMT_Q4_K> {
   static constexpr int PIECES(int WN) { return WN * RAW / 1024; }
   struct St {
     u32x4 q;
+    u32x2 s;
     float D0, M0, D1, M1;
   };
-  LA_DEV static void load(const uint8_t* raw, const uint8_t* scl, int c, int h, int, St& st) {
+  LA_DEV static void fetch(const uint8_t* raw, const uint8_t* scl, int c, int h, int, St& st) {
     st.q = *(const u32x4*)(raw + c * 32 + 16 * (h ^ ((c >> 3) & 1)));
-    const u32x2 s = *(const u32x2*)(scl + c * 8);  // f16 D0, -M0, D1, -M1 (la_gemm_scales)
-    st.D0 = h2f(s.x & 0xFFFFu);
-    st.M0 = h2f(s.x >> 16);
-    st.D1 = h2f(s.y & 0xFFFFu);
-    st.M1 = h2f(s.y >> 16);
+    st.s = *(const u32x2*)(scl + c * 8);  // f16 D0, -M0, D1, -M1 (la_gemm_scales)
+  }
+  LA_DEV static void pin(St& st) { q32_pin(st.q), q32_pin(st.s); }
+  LA_DEV static void prep(St& st, int) {
+    st.D0 = 512.f * h2f(st.s.x & 0xFFFFu);   // see deq
+    st.M0 = h2f(st.s.x >> 16);
+    st.D1 = 512.f * h2f(st.s.y & 0xFFFFu);
+    st.M1 = h2f(st.s.y >> 16);
+  }
+  LA_DEV static void load(const uint8_t* raw, const uint8_t* scl, int c, int h, int ks, St& st) {
+    fetch(raw, scl, c, h, ks, st);
+    prep(st, h);
   }
   template <int S>
   LA_DEV static bf16x8 deq(const St& st) {
+    typedef float f32x2 __attribute__((ext_vector_type(2)));
     const uint32_t w0 = (S & 1) ? st.q.z : st.q.x, w1 = (S & 1) ? st.q.w : st.q.y;
-    uint32_t lo, hi;
-    // opaque masks: one v_cvt_f32_ubyteN per weight (a packed v_cvt_pk_f32_fp8 + v_pk_fma_f32 form,
-    // 1.75 VALU per weight, was no faster on moe32 / the C=256 step and miscomputed the 64-column
-    // variants: profiles/r6_moe_live.md)
-    if constexpr (S < 2) {
-      asm("v_and_b32 %0, 0x0f0f0f0f, %1" : "=v"(lo) : "v"(w0));
-      asm("v_and_b32 %0, 0x0f0f0f0f, %1" : "=v"(hi) : "v"(w1));
-    } else {
-      asm("v_and_b32 %0, 0x0f0f0f0f, %1" : "=v"(lo) : "v"(w0 >> 4));
-      asm("v_and_b32 %0, 0x0f0f0f0f, %1" : "=v"(hi) : "v"(w1 >> 4));
-    }
+    // codes 0 .. 15 read as fp8 e4m3 are exactly code / 512: two a v_cvt_pk_f32_fp8 (2.5 VALU per weight, not 2.9)
+    const uint32_t lo = (w0 >> (4 * (S >> 1))) & 0x0F0F0F0Fu, hi = (w1 >> (4 * (S >> 1))) & 0x0F0F0F0Fu;
     const float D = S < 2 ? st.D0 : st.D1, Mn = S < 2 ? st.M0 : st.M1;
-    bf16x8 r;
-#pragma unroll
-    for (int b = 0; b < 4; ++b) {
-      r[b] = (bf16)fmaf(D, (float)((lo >> (8 * b)) & 0xFFu), Mn);
-      r[b + 4] = (bf16)fmaf(D, (float)((hi >> (8 * b)) & 0xFFu), Mn);
-    }
-    return r;
+    const f32x2 a0 = __builtin_amdgcn_cvt_pk_f32_fp8(lo, false), a1 = __builtin_amdgcn_cvt_pk_f32_fp8(lo, true);
+    const f32x2 b0 = __builtin_amdgcn_cvt_pk_f32_fp8(hi, false), b1 = __builtin_amdgcn_cvt_pk_f32_fp8(hi, true);
+    const u32x4 v = {pk_bf16(fmaf(D, a0.x, Mn), fmaf(D, a0.y, Mn)), pk_bf16(fmaf(D, a1.x, Mn), fmaf(D, a1.y, Mn)),
+                     pk_bf16(fmaf(D, b0.x, Mn), fmaf(D, b0.y, Mn)), pk_bf16(fmaf(D, b1.x, Mn), fmaf(D, b1.y, Mn))};
+    return __builtin_bit_cast(bf16x8, v);
   }
 };
 
@@ -149,19 +153,27 @@ template <> struct Q32F<FMT_Q6_K> {
   }
   struct St {
     u32x4 ql, qh;
+    u32x2 s;
     float S0, S1;
     int sh;
   };
+  LA_DEV static void pin(St& st) { q32_pin(st.ql), q32_pin(st.qh), q32_pin(st.s); }
   // raw layout per wave: piece 2cb = ql of columns 32cb.., piece 2cb+1 = qh of the same columns
-  LA_DEV static void load(const uint8_t* raw, const uint8_t* scl, int c, int h, int ks, St& st) {
+  LA_DEV static void fetch(const uint8_t* raw, const uint8_t* scl, int c, int h, int ks, St& st) {
     const int cb = c >> 5, cl = c & 31;
     const int o = cl * 32 + 16 * (h ^ ((cl >> 3) & 1));
     st.ql = *(const u32x4*)(raw + (2 * cb) * 1024 + o);
     st.qh = *(const u32x4*)(raw + (2 * cb + 1) * 1024 + o);
-    const u32x2 s = *(const u32x2*)(scl + c * 8);  // f16 d*sc: run0 g0, run0 g1, run1 g0, run1 g1
-    st.S0 = h2f(h ? (s.x >> 16) : (s.x & 0xFFFFu));
-    st.S1 = h2f(h ? (s.y >> 16) : (s.y & 0xFFFFu));
+    st.s = *(const u32x2*)(scl + c * 8);  // f16 d*sc: run0 g0, run0 g1, run1 g0, run1 g1
     st.sh = 2 * (ks & 1);
+  }
+  LA_DEV static void prep(St& st, int h) {
+    st.S0 = h2f(h ? (st.s.x >> 16) : (st.s.x & 0xFFFFu));
+    st.S1 = h2f(h ? (st.s.y >> 16) : (st.s.y & 0xFFFFu));
+  }
+  LA_DEV static void load(const uint8_t* raw, const uint8_t* scl, int c, int h, int ks, St& st) {
+    fetch(raw, scl, c, h, ks, st);
+    prep(st, h);
   }
   template <int S>
   LA_DEV static bf16x8 deq(const St& st) {
@@ -204,15 +216,23 @@ template <> struct Q32F<FMT_Q8_0> {
   }
   struct St {
     u32x4 q0, q1;
+    uint32_t s;
     float d, o;
   };
-  LA_DEV static void load(const uint8_t* raw, const uint8_t* scl, int c, int h, int, St& st) {
+  LA_DEV static void pin(St& st) { q32_pin(st.q0), q32_pin(st.q1), q32_pin(st.s); }
+  LA_DEV static void fetch(const uint8_t* raw, const uint8_t* scl, int c, int h, int, St& st) {
     const int sw = (c >> 2) & 3;
     st.q0 = *(const u32x4*)(raw + c * 64 + 16 * ((2 * h) ^ sw));
     st.q1 = *(const u32x4*)(raw + c * 64 + 16 * ((2 * h + 1) ^ sw));
-    const uint32_t s = *(const uint32_t*)(scl + c * 8);  // f16 d0, d1
-    st.d = h2f(h ? (s >> 16) : (s & 0xFFFFu));
+    st.s = *(const uint32_t*)(scl + c * 8);  // f16 d0, d1
+  }
+  LA_DEV static void prep(St& st, int h) {
+    st.d = h2f(h ? (st.s >> 16) : (st.s & 0xFFFFu));
     st.o = -128.0f * st.d;
+  }
+  LA_DEV static void load(const uint8_t* raw, const uint8_t* scl, int c, int h, int ks, St& st) {
+    fetch(raw, scl, c, h, ks, st);
+    prep(st, h);
   }
   template <int S>
   LA_DEV static bf16x8 deq(const St& st) {
@@ -267,6 +287,123 @@ struct Q32Moe {
 };
 
 LA_DEV float q32_gelu_tanh(float x) { return 0.5f * x * (1.f + tanhf(0.7978845608f * (x + 0.044715f * x * x * x))); }
+
+// The K loop in sub-steps of 16 k: the products of one run beside the dequantisation of the next (an MFMA, then its share
+// of the vector instructions), with one fragment set in use and one being read.  A wave's raw bytes are its own, so
+// they are read after its own vmcnt; the barrier that makes the next stage's X visible and this stage's slot free stands
+// before the last sub-step, whose DMA goes between its MFMAs.  The last NS stages issue the final one again: the counts
+// stay constants and the loop has no branch.
+template <int FMT, int BM, int WN, int NS, int NW, int MBL, bool OK, int PX, int PS, int MB, int CB>
+LA_DEV void q32_loop2(uint8_t* lds, const bf16* X, const Q32Cols& cm, const uint32_t (&xoff)[PX], const uint8_t* const (&srec)[PS],
+                      const int (&aoff)[4], int ks0, int nk, int wave, int lane, f32x16_t (&acc)[MB][CB]) {
+  static_assert(OK, "no probe of this schedule");
+  using F = Q32F<FMT>;
+  using G = Q32Geo<FMT, BM, WN, NW>;
+  constexpr int NM = MBL * CB, VPM = (22 * CB + NM - 1) / NM;
+  const int r32 = lane & 31, h = lane >> 5;
+  auto issue = [&](int t, int slot) {
+    const int ks = ks0 + min(t, nk - 1);
+    uint8_t* sl = lds + slot * G::SLOT;
+    const uint8_t* xk = (const uint8_t*)(X + F::xk(ks));
+#pragma unroll
+    for (int j = 0; j < PX; ++j) q32_glds16(xk + 2 * (size_t)xoff[j], sl + (wave * PX + j) * 1024);
+    uint8_t* rw = sl + G::XB + wave * G::RW;
+#pragma unroll
+    for (int p = 0; p < G::PR; ++p) F::issue(cm, ks, p, rw, lane);
+    uint8_t* sw = sl + G::XB + NW * G::RW + wave * G::SW;
+#pragma unroll
+    for (int p = 0; p < PS; ++p) q32_glds4(srec[p] + (size_t)ks * 128, sw + p * 256);
+  };
+  auto read_a = [&](u32x4 (&a)[MBL], int slot, int s) {
+    const uint8_t* sl = lds + slot * G::SLOT;
+#pragma unroll
+    for (int mb = 0; mb < MBL; ++mb) a[mb] = *(const u32x4*)(sl + mb * 4096 + aoff[s]);
+  };
+  auto pin_a = [&](u32x4 (&a)[MBL]) {
+#pragma unroll
+    for (int mb = 0; mb < MBL; ++mb) q32_pin(a[mb]);
+  };
+  auto fetch = [&](typename F::St (&st)[CB], int t, int slot) {
+    const uint8_t* sl = lds + slot * G::SLOT + G::XB;
+#pragma unroll
+    for (int cb = 0; cb < CB; ++cb)
+      F::fetch(sl + wave * G::RW, sl + NW * G::RW + wave * G::SW, cb * 32 + r32, h, ks0 + t, st[cb]);
+  };
+  auto deq = [&](bf16x8 (&b)[CB], const typename F::St (&st)[CB], auto S) {
+#pragma unroll
+    for (int cb = 0; cb < CB; ++cb) b[cb] = F::template deq<decltype(S)::value>(st[cb]);
+  };
+  auto mul = [&](const u32x4 (&a)[MBL], const bf16x8 (&b)[CB], auto dma) {
+#pragma unroll
+    for (int mb = 0; mb < MBL; ++mb)
+#pragma unroll
+      for (int cb = 0; cb < CB; ++cb)
+        acc[mb][cb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a[mb]), b[cb], acc[mb][cb], 0, 0, 0);
+#pragma unroll
+    for (int i = 0; i < NM; ++i) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(0x002, VPM, 0);
+      if (decltype(dma)::value) __builtin_amdgcn_sched_group_barrier(0x010, 1, 0);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  using S0 = std::integral_constant<int, 0>;
+  using S1 = std::integral_constant<int, 1>;
+  using S2 = std::integral_constant<int, 2>;
+  using S3 = std::integral_constant<int, 3>;
+#pragma unroll
+  for (int i = 0; i < NS; ++i) issue(i, i);
+  q32_vmwait<(NS - 1) * G::L>();
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+  u32x4 a0[MBL], a1[MBL];
+  bf16x8 b0[CB], b1[CB];
+  typename F::St sa[CB], sb[CB];
+  fetch(sa, 0, 0);
+  read_a(a0, 0, 0);
+#pragma unroll
+  for (int cb = 0; cb < CB; ++cb) F::prep(sa[cb], h);
+  deq(b0, sa, S0{});
+  int slot = 0;
+  auto step = [&](typename F::St (&cur)[CB], typename F::St (&nxt)[CB], int t) {
+    const int next = slot == NS - 1 ? 0 : slot + 1;
+    pin_a(a0);
+    read_a(a1, slot, 1);
+    __builtin_amdgcn_sched_barrier(0);
+    deq(b1, cur, S1{});
+    mul(a0, b0, std::false_type{});
+    pin_a(a1);
+    read_a(a0, slot, 2);
+    __builtin_amdgcn_sched_barrier(0);
+    deq(b0, cur, S2{});
+    mul(a1, b1, std::false_type{});
+    pin_a(a0);
+    q32_vmwait<(NS - 2) * G::L>();             // this wave's part of stage t + 1
+    fetch(nxt, t + 1, next);
+    read_a(a1, slot, 3);
+    __builtin_amdgcn_sched_barrier(0);
+    deq(b1, cur, S3{});
+    mul(a0, b0, std::false_type{});
+    pin_a(a1);
+#pragma unroll
+    for (int cb = 0; cb < CB; ++cb) F::pin(nxt[cb]);
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    read_a(a0, next, 0);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int cb = 0; cb < CB; ++cb) F::prep(nxt[cb], h);
+    deq(b0, nxt, S0{});
+    issue(t + NS, slot);
+    mul(a1, b1, std::true_type{});
+    slot = next;
+  };
+  for (int t = 0; t + 1 < nk; t += 2) {
+    step(sa, sb, t);
+    step(sb, sa, t + 1);
+  }
+  if (nk & 1) step(sa, sb, nk - 1);
+  q32_vmwait<0>();                              // nothing may land in the epilogue's images
+}
 
 // One (M tile, N tile, K split).  GLU: columns [0, BN/2) of the tile are gate rows, [BN/2, BN)
 // the matching up rows; no split.
@@ -412,6 +549,9 @@ LA_DEV void q32_tile(uint8_t* __restrict__ lds, const QW& w, int tile, const bf1
     read_a(alo, t + 1, 0);
   };
 
+  if constexpr (PIPE == 2) {
+    q32_loop2<FMT, BM, WN, NS, NW_, MBL, (ABL == 0)>(lds, X, cm, xoff, srec, aoff, ks0, nk, wave, lane, acc);
+  } else {
   bf16x8 alo[2][MB], ahi[2][MB];
   typename F::St st[CB];
   // prologue: all NS slots in flight, then stage 0's B and A sub-steps 0, 1 into registers
@@ -498,6 +638,7 @@ LA_DEV void q32_tile(uint8_t* __restrict__ lds, const QW& w, int tile, const bf1
       mm(ahi[0], b2);
       mm(ahi[1], b3);
     }
+  }
   }
 
   // ---- epilogue through LDS: acc[mb][cb] reg j = (row mb*32 + (j&3) + 8(j>>2) + 4h, col cb*32 + r32)
@@ -658,7 +799,9 @@ __global__ __launch_bounds__(C::NW * 64, 1) __attribute__((amdgpu_waves_per_eu(C
 
 // variant ids (shared with ops/__init__.py Q32_VARIANTS): tile BM x BN, waves, schedule
 //   0: 256 x 128 (4 waves)   1: 128 x 256 (4)   2: 256 x 256 (4)   3: 128 x 128 (4)
-//   8: 128 x 256 (8 waves, 2 per SIMD);  +4 (4 .. 7) / 9: the same with the interleaved schedule (PIPE = 1)
+//   8: 128 x 256 (8 waves, 2 per SIMD);  5 .. 7: 1 .. 3 with the interleaved schedule (PIPE = 1);  4, 9: 0 and 8 with
+//   the sub-step schedule (PIPE = 2; 4096 x 14336 of Q4_K in 8 splits: 256 rows 46 -> 44 and 50 -> 47 us, 96 rows 41.5 ->
+//   38; gate|up 28672 x 4096 in variant 9: 128 rows 76 -> 67)
 // The 256 x 256 tiles (2, 6) hold 256 accumulator registers per lane: Q4_K only (the larger
 // Q6_K / Q8_0 fragment state does not fit beside them without spilling).
 template <bool BIG, class Fn>
@@ -671,11 +814,11 @@ static int q32_var(int var, Fn&& fn) {
     case 0: fn(Q32Cfg<256, 32, 4, 0>{}); break;
     case 1: fn(Q32Cfg<128, 64, 4, 0>{}); break;
     case 3: fn(Q32Cfg<128, 32, 4, 0>{}); break;
-    case 4: fn(Q32Cfg<256, 32, 4, 1>{}); break;
+    case 4: fn(Q32Cfg<256, 32, 4, 2>{}); break;
     case 5: fn(Q32Cfg<128, 64, 4, 1>{}); break;
     case 7: fn(Q32Cfg<128, 32, 4, 1>{}); break;
     case 8: fn(Q32Cfg<128, 32, 8, 0>{}); break;
-    case 9: fn(Q32Cfg<128, 32, 8, 1>{}); break;
+    case 9: fn(Q32Cfg<128, 32, 8, 2>{}); break;
     default: return -1;
   }
   return 0;
@@ -838,8 +981,11 @@ static int moe32_var(int var, Fn&& fn) {
     case 17: fn(MoeCfg<Q32Cfg<64, 32, 8, 0>, 2, 0, true>{}); break;
     case 18: fn(MoeCfg<Q32Cfg<128, 32, 4, 1>, 1, 0, true>{}); break;
     // 64 columns per wave: twice the weight bytes per ring stage against the same X stage (the
-    // 128-row X slab is most of a stage), so twice the weight bytes in flight per CU
-    case 19: if constexpr (Q4) fn(MoeCfg<Q32Cfg<128, 64, 8, 0>, 1, 0, true>{}); else return -1; break;
+    // 128-row X slab is most of a stage), so twice the weight bytes in flight per CU.  In the sub-step schedule, which
+    // fits Q6_K and Q8_0 too: 8 experts of 28672 | 14336 x 4096, top 2, 1203 tokens 1305 -> 1150 us a layer (Q6_K down);
+    // with the products in one block and the dequantisation in another each waited for the other.  Variants 9 and 17
+    // (fewer rows: bound by the weight bytes) gained nothing from it
+    case 19: fn(MoeCfg<Q32Cfg<128, 64, 8, 2>, 1, 0, true>{}); break;
     case 20: if constexpr (Q4) fn(MoeCfg<Q32Cfg<128, 64, 4, 0>, 1, 0, true>{}); else return -1; break;
     default: return -1;
   }
@@ -853,7 +999,7 @@ static int moe32_launch(int var, const QW* qws, int N, int K, int E, const int* 
   const int KS = K >> 6, per = (KS + splits - 1) / splits;
   // 64 columns per wave at 128 rows spill with Q6_K / Q8_0's larger fragment state: those formats
   // take the 32-column form of the same chunking
-  if (FMT != FMT_Q4_K && (var == 19 || var == 20)) var -= 4;
+  if (FMT != FMT_Q4_K && var == 20) var -= 4;
   return moe32_var<FMT == FMT_Q4_K>(var, [&](auto c) {
     using C = decltype(c);
     const int mch = (maxM + C::BM - 1) / C::BM;
