@@ -365,6 +365,9 @@ __global__ __launch_bounds__(256) void rope_kv_kernel(Src qkv, const int* __rest
 // thread per 8 consecutive elements of a row (16-byte source loads, two float4 cos/sin loads,
 // 16-byte q / k stores; the 8 V values of a unit land in one 128-byte line of the grouped-
 // transposed V page).  The block's token position and slot are read once.
+// R rows a workgroup.  Bound by the bytes (8192 rows of 6144: 200 MB, 44.7 us) where R is 4: V's lines hold eight keys,
+// and written two bytes a key by workgroups on different XCDs they cost as much as half of the rest, so a prompt's rows
+// go there by the eight; with one row a workgroup the loads' latency is the bound and the longer chain is not worth it.
 LA_DEV void load8(const Src& s, long idx, int col, float v[8]) {
   if (s.S == 0) {
     const bf16x8 b = *(const bf16x8*)((const bf16*)s.p + idx);
@@ -381,47 +384,80 @@ LA_DEV void load8(const Src& s, long idx, int col, float v[8]) {
   }
 }
 
-template <int DH>
+template <int DH, int R>
 __global__ __launch_bounds__(256) void rope_kv8_kernel(Src qkv, const int* __restrict__ pos,
                                                        const int* __restrict__ slots,
-                                                       const float* __restrict__ cos_sin, int Hq, int Hkv,
+                                                       const float* __restrict__ cos_sin, int T, int Hq, int Hkv,
                                                        bf16* __restrict__ q_out, bf16* __restrict__ kc,
                                                        bf16* __restrict__ vc, int BS) {
-  const int t = blockIdx.x;
+  const int tb = blockIdx.x * R;
   const int W = (Hq + 2 * Hkv) * DH;
-  const int p = pos[t];
-  const int slot = slots ? slots[t] : -1;
-  const long row = (long)t * W;
-  const float* cs = cos_sin + (long)p * DH;  // DH/2 pairs x (cos, sin)
-  const int units = W >> 3;
   const int u = blockIdx.y * blockDim.x + threadIdx.x;
-  if (u >= units) return;
+  if (u >= W >> 3) return;
   const int col = u * 8;
   const int head = col / DH, d0 = col - head * DH;
-  float v[8];
-  load8(qkv, row + col, col, v);
   if (head >= Hq + Hkv) {  // v: no rotation
-    if (slot < 0) return;
-    const int vh = head - Hq - Hkv, blk = slot / BS, off = slot - blk * BS;
-    bf16* dst = vc + ((long)blk * Hkv + vh) * DH * BS + ((off >> 3) * DH + d0) * 8 + (off & 7);
+    const int vh = head - Hq - Hkv;
+#pragma unroll 1
+    for (int t = tb; t < min(tb + R, T); ++t) {
+      float v[8];
+      if (R == 1) load8(qkv, (long)t * W + col, col, v);   // beside the slot's load, not behind it
+      const int slot = slots ? slots[t] : -1;
+      if (slot < 0) continue;
+      const int blk = slot / BS, off = slot - blk * BS, e = off & 7, t0 = t - e;
+      bf16* dst = vc + ((long)blk * Hkv + vh) * DH * BS + ((off >> 3) * DH + d0) * 8;
+      // eight rows that fill one group of eight keys (a prompt's): the first writes all of them, 128 bytes a thread
+      bool whole = R > 1 && t0 >= 0 && t0 + 7 < T;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) dst[8 * j] = (bf16)v[j];
+      for (int i = 0; R > 1 && i < 8; ++i) whole &= slots[min(max(t0 + i, 0), T - 1)] == slot - e + i;
+      if (whole && e) continue;
+      if (whole) {
+        float x[8][8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) load8(qkv, (long)(t + i) * W + col, col, x[i]);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          bf16x8 g;
+#pragma unroll
+          for (int i = 0; i < 8; ++i) g[i] = (bf16)x[i][j];
+          *(bf16x8*)(dst + 8 * j) = g;
+        }
+      } else {
+        if (R > 1) load8(qkv, (long)t * W + col, col, v);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) dst[8 * j + e] = (bf16)v[j];
+      }
+    }
     return;
   }
-  const float4 c0 = *(const float4*)(cs + d0), c1 = *(const float4*)(cs + d0 + 4);  // pairs d0/2 .. d0/2+3
-  const float cc[4] = {c0.x, c0.z, c1.x, c1.z}, sn[4] = {c0.y, c0.w, c1.y, c1.w};
-  bf16x8 o;
+  int slot[R];
+  float v[R][8];
+  float4 c0[R], c1[R];
 #pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const float x0 = v[2 * j], x1 = v[2 * j + 1];
-    o[2 * j] = (bf16)(x0 * cc[j] - x1 * sn[j]);
-    o[2 * j + 1] = (bf16)(x0 * sn[j] + x1 * cc[j]);
+  for (int r = 0; r < R; ++r) {
+    const int t = min(tb + r, T - 1);
+    const float* cs = cos_sin + (long)pos[t] * DH + d0;  // DH/2 pairs x (cos, sin): d0/2 .. d0/2+3
+    load8(qkv, (long)t * W + col, col, v[r]);
+    slot[r] = slots ? slots[t] : -1;
+    c0[r] = *(const float4*)cs, c1[r] = *(const float4*)(cs + 4);
   }
-  if (head < Hq) {
-    *(bf16x8*)(q_out + ((long)t * Hq + head) * DH + d0) = o;
-  } else if (slot >= 0) {
-    const int kh = head - Hq, blk = slot / BS, off = slot - blk * BS;
-    *(bf16x8*)(kc + (((long)blk * Hkv + kh) * BS + off) * DH + d0) = o;
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    if (tb + r >= T) break;
+    const float cc[4] = {c0[r].x, c0[r].z, c1[r].x, c1[r].z}, sn[4] = {c0[r].y, c0[r].w, c1[r].y, c1[r].w};
+    bf16x8 o;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const float x0 = v[r][2 * j], x1 = v[r][2 * j + 1];
+      o[2 * j] = (bf16)(x0 * cc[j] - x1 * sn[j]);
+      o[2 * j + 1] = (bf16)(x0 * sn[j] + x1 * cc[j]);
+    }
+    if (head < Hq) {
+      *(bf16x8*)(q_out + ((long)(tb + r) * Hq + head) * DH + d0) = o;
+    } else if (slot[r] >= 0) {
+      const int kh = head - Hq, blk = slot[r] / BS, off = slot[r] - blk * BS;
+      *(bf16x8*)(kc + (((long)blk * Hkv + kh) * BS + off) * DH + d0) = o;
+    }
   }
 }
 
@@ -651,15 +687,20 @@ extern "C" int la_rope_kv(const void* qkv_p, long slab, int S, const void* bias,
                           void* kc, void* vc, int BS, void* stream) {
   if ((Dh & 3) || (rot & 3) || rot > Dh) return -1;
   Src s{qkv_p, slab, S, (const float*)bias};
-  if (mode == 0 && rot == Dh && (Dh == 128 || Dh == 64) && (BS & 7) == 0) {
+  if (mode == 0 && rot == Dh && (Dh == 128 || Dh == 64) && (BS & 7) == 0 && ((uintptr_t)vc & 15) == 0) {
     const int units8 = (Hq + 2 * Hkv) * Dh / 8;
-    dim3 grid(T, (units8 + 255) / 256);
-    if (Dh == 128)
-      hipLaunchKernelGGL(la::rope_kv8_kernel<128>, grid, dim3(256), 0, (hipStream_t)stream, s, pos, slots, cos_sin,
-                         Hq, Hkv, (bf16*)q_out, (bf16*)kc, (bf16*)vc, BS);
-    else
-      hipLaunchKernelGGL(la::rope_kv8_kernel<64>, grid, dim3(256), 0, (hipStream_t)stream, s, pos, slots, cos_sin,
-                         Hq, Hkv, (bf16*)q_out, (bf16*)kc, (bf16*)vc, BS);
+    // Four rows a workgroup once that leaves two workgroups for every CU: a row is a chain of three loads.  Rows of 6144,
+    // one against four: 300 rows 6.8 / 8.4 us, 701 10.1 / 7.7, 1203 15.5 / 11.8, 2048 21.9 / 15.1, 8192 67 / 44.7
+    const int R = (long)T * ((units8 + 255) / 256) >= 2048 ? 4 : 1;
+    dim3 grid((T + R - 1) / R, (units8 + 255) / 256);
+#define LA_ROPE8(D, R_)                                                                                              \
+  hipLaunchKernelGGL((la::rope_kv8_kernel<D, R_>), grid, dim3(256), 0, (hipStream_t)stream, s, pos, slots, cos_sin, T, \
+                     Hq, Hkv, (bf16*)q_out, (bf16*)kc, (bf16*)vc, BS)
+    if (Dh == 128 && R == 4) LA_ROPE8(128, 4);
+    else if (Dh == 128) LA_ROPE8(128, 1);
+    else if (R == 4) LA_ROPE8(64, 4);
+    else LA_ROPE8(64, 1);
+#undef LA_ROPE8
     return (int)hipGetLastError();
   }
   const int units = (Hq + 2 * Hkv) * Dh / 4;

@@ -194,3 +194,29 @@ def test_prompt_plan(t, N, K, M, tile):
         s, u = torch.nn.functional.silu(ref[:, :N // 2]), ref[:, N // 2:]
         eg, eu = bound[:, :N // 2], bound[:, N // 2:]
         assert ((h.float() - s * u).abs() <= 1.2 * eg * (u.abs() + eu) + s.abs() * eu + 2 ** -8 * (s * u).abs() + 1e-5).all()
+
+
+@pytest.mark.parametrize("T,BS,Dh,S", [(37, 16, 128, 0), (64, 8, 64, 0), (200, 64, 128, 3), (9, 32, 64, 1), (1501, 16, 128, 0)])
+def test_rope_rows_of_a_prompt(T, BS, Dh, S):
+    """Rows that fill groups of eight keys, with runs that begin inside one, end inside one, skip a row or are not stored:
+    bit for bit what each row alone writes."""
+    Hq, Hkv = 4, 2
+    W, g = (Hq + 2 * Hkv) * Dh, torch.Generator().manual_seed(T)
+    x = torch.randn(max(S, 1), T, W, generator=g).to(DEV)
+    x = x if S else x[0].to(torch.bfloat16)
+    slots, at = torch.empty(T, dtype=torch.int32), 3
+    for t in range(T):                       # a new run of slots every 23 rows, a row of padding now and then
+        at = at + 1 if t % 23 else at + 5
+        slots[t] = -1 if t % 19 == 17 else at
+    nb = at // BS + 2
+    pos = torch.arange(T, dtype=torch.int32)
+    cs = torch.randn(T, Dh, generator=g).to(DEV)
+    kc = torch.zeros(nb, Hkv, BS, Dh, dtype=torch.bfloat16, device=DEV)
+    one = [kc, torch.zeros(nb, Hkv, BS // 8, Dh, 8, dtype=torch.bfloat16, device=DEV)]
+    many = [c.clone() for c in one]
+    q1 = [ops.rope_kv(ops.Partial(x[..., t:t + 1, :].contiguous()), pos[t:t + 1].to(DEV), slots[t:t + 1].to(DEV), cs, Hq, Hkv, Dh, Dh, 0,
+                      *one, BS) for t in range(T)]
+    q = ops.rope_kv(ops.Partial(x), pos.to(DEV), slots.to(DEV), cs, Hq, Hkv, Dh, Dh, 0, *many, BS)
+    assert torch.equal(q.view(T, -1), torch.cat([a.view(1, -1) for a in q1]))
+    assert torch.equal(one[0], many[0]) and torch.equal(one[1], many[1])
+    assert one[1].abs().sum() > 0
