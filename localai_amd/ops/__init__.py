@@ -93,6 +93,7 @@ def lib():
             "la_dequant": [I, P, P, P, P, I, I, P, P],
             "la_attn_decode": [P, P, P, P, I, P, I, I, I, I, I, F, I, I, P, P, P, P, P, LNG, I, P, P, P, P, F, I, I, P, I, P,
                                P, I, P, LNG, I, P],
+            "la_attn_prefill_split": [P, P, P, P, I, P, P, P, I, I, I, I, I, F, P, I, I, P, P],
             "la_attn_prefill": [P, P, P, P, I, P, P, P, I, I, I, I, I, F, P, F, I, P, I, P, P, I, P, LNG, I, P],
             "la_sample": [P, LNG, I, I, P, P, P, P, P],
             "la_penalties": [P, LNG, I, P, I, P, P, I, P, P],
@@ -1867,6 +1868,17 @@ def prefill_tiles(q_lens: Sequence[int], device) -> torch.Tensor:
     return torch.tensor(tiles, dtype=torch.int32, device=device).view(-1, 2)
 
 
+def _prefill_splits(ntiles: int, Hq: int, Hkv: int, Dh: int, BS: int, keys: int, rows: int) -> int:
+    """Workgroups that share one work tile's keys in attn_prefill (sequences of up to `keys` keys, `rows` of them new):
+    enough for two workgroups on every CU, each with 256 keys or more on average.  32 heads over 8, one against the
+    split (us): 16 rows behind 2000 keys 56 / 16, 100 behind 8000 215 / 38, 300 behind 12000 322 / 101, 700 behind 4000
+    134 / 104, 4 times 50 behind 3000 86 / 36; past the line 701 rows alone 25 / 33, 2048 behind 10007 457 / 507."""
+    if Dh not in (64, 128) or BS < 16 or BS & (BS - 1) or ntiles < 1:
+        return 1
+    groups = ntiles * (Hq if (Hq // Hkv) % 2 else Hq // 2)
+    return max(1, min(16, 512 // groups, (keys - rows // 2) // 256))
+
+
 def attn_prefill(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, cu_q: torch.Tensor,
                  ctx_lens: torch.Tensor, block_tables: torch.Tensor, scale: float,
                  tiles: Optional[torch.Tensor] = None, q_lens: Optional[Sequence[int]] = None,
@@ -1888,6 +1900,16 @@ def attn_prefill(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, 
         tiles = prefill_tiles([cq[i + 1] - cq[i] for i in range(len(cq) - 1)], q.device)
     if out is None:
         out = torch.empty(T, Hq, Dh, dtype=torch.bfloat16, device=q.device)
+    plain = dist_bias is None and sink is None and sigmoid_bias is None and not chunk and gate is None and not keep and softcap <= 0 and window <= 0
+    P = _prefill_splits(tiles.shape[0], Hq, Hkv, Dh, k_cache.shape[2], block_tables.shape[1] * k_cache.shape[2],
+                        T // max(1, ctx_lens.shape[0])) if plain and scale > 0 else 1
+    if P > 1:
+        ws = torch.empty(P * T * Hq * (Dh + 2), dtype=torch.float32, device=q.device)
+        _check(lib().la_attn_prefill_split(q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), tiles.data_ptr(), tiles.shape[0],
+                                           cu_q.data_ptr(), ctx_lens.data_ptr(), block_tables.data_ptr(), block_tables.shape[1],
+                                           Hq, Hkv, Dh, k_cache.shape[2], float(scale), out.data_ptr(), T, P, ws.data_ptr(),
+                                           _stream()), "la_attn_prefill_split")
+        return out
     _check(lib().la_attn_prefill(q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), tiles.data_ptr(),
                                  tiles.shape[0], cu_q.data_ptr(), ctx_lens.data_ptr(), block_tables.data_ptr(),
                                  block_tables.shape[1], Hq, Hkv, Dh, k_cache.shape[2], float(scale),

@@ -879,6 +879,32 @@ static int flash_heads(int ntiles, int Hq, int G, long keys) {
   return G % 2 ? 1 : 2;
 }
 
+// The plain causal form with every work tile's keys split over P workgroups; ws: P * T * Hq * (Dh + 2) floats.
+extern "C" int la_attn_prefill_split(const void* q, const void* kc, const void* vc, const int* tiles, int ntiles,
+                                     const int* cu_q, const int* ctx_lens, const int* block_tables, int max_blocks, int Hq,
+                                     int Hkv, int Dh, int BS, float scale, void* out, int T, int P, void* ws, void* stream) {
+  if (Hkv < 1 || Hq % Hkv || (Dh != 64 && Dh != 128) || !(scale > 0.f) || BS < 16 || (BS & (BS - 1)) || ntiles < 1 ||
+      ntiles > 65535 || T < 1 || P < 1 || P > 64 || !ws || ((uintptr_t)ws & 15))
+    return -1;
+  hipStream_t st = (hipStream_t)stream;
+  const int hpw = (Hq / Hkv) % 2 ? 1 : 2;
+  const long n = (long)P * T * Hq;
+  const la::FlashSplit sp{(float*)ws, (float2*)((float*)ws + n * Dh), T};
+  const dim3 fg(Hq / hpw, ntiles, P);
+#define FL(D, H)                                                                                                    \
+  hipLaunchKernelGGL((la::prefill_flash_kernel<D, H, true>), fg, dim3(H * 128), 0, st, (const bf16*)q,              \
+                     (const bf16*)kc, (const bf16*)vc, tiles, cu_q, ctx_lens, block_tables, max_blocks, Hq, Hkv,    \
+                     __builtin_ctz(BS), scale * 1.4426950408889634f, (bf16*)out, sp)
+  if (Dh == 128 && hpw == 2) FL(128, 2);
+  else if (Dh == 128) FL(128, 1);
+  else if (hpw == 2) FL(64, 2);
+  else FL(64, 1);
+#undef FL
+  if (Dh == 128) hipLaunchKernelGGL(la::flash_merge_kernel<128>, dim3(Hq, ntiles, la::FL_QT / 8), dim3(256), 0, st, sp, P, tiles, cu_q, Hq, (bf16*)out);
+  else hipLaunchKernelGGL(la::flash_merge_kernel<64>, dim3(Hq, ntiles, la::FL_QT / 16), dim3(256), 0, st, sp, P, tiles, cu_q, Hq, (bf16*)out);
+  return (int)hipGetLastError();
+}
+
 extern "C" int la_attn_prefill(const void* q, const void* kc, const void* vc, const int* tiles, int ntiles,
                                const int* cu_q, const int* ctx_lens, const int* block_tables, int max_blocks, int Hq,
                                int Hkv, int Dh, int BS, float scale, void* out, float softcap, int window,
@@ -896,9 +922,9 @@ extern "C" int la_attn_prefill(const void* q, const void* kc, const void* vc, co
     const dim3 fg(Hq / hpw, ntiles);
     const int shift = __builtin_ctz(BS);
 #define FL(D, H)                                                                                                  \
-  hipLaunchKernelGGL((la::prefill_flash_kernel<D, H>), fg, dim3(H * 128), 0, st, (const bf16*)q, (const bf16*)kc, \
-                     (const bf16*)vc, tiles, cu_q, ctx_lens, block_tables, max_blocks, Hq, Hkv, shift,            \
-                     scale * 1.4426950408889634f, (bf16*)out)
+  hipLaunchKernelGGL((la::prefill_flash_kernel<D, H, false>), fg, dim3(H * 128), 0, st, (const bf16*)q,            \
+                     (const bf16*)kc, (const bf16*)vc, tiles, cu_q, ctx_lens, block_tables, max_blocks, Hq, Hkv,   \
+                     shift, scale * 1.4426950408889634f, (bf16*)out, la::FlashSplit{})
 #define FL_H(D)                \
   do {                         \
     if (hpw == 4) FL(D, 4);    \

@@ -18,7 +18,10 @@
 // 2048 rows behind 10007 keys, 32 heads over 8, width 128: 3233 us with the 64 x 32 tile of one head that
 // attn_prefill_kernel takes (114 TFLOP/s), 451 us here (821); one prompt of 701 tokens 96 -> 26 us; 64 of 128 164 -> 51.
 // A third schedule, with the next tile's score product between the exponentials, was 5 % slower (V arrives one half
-// iteration later, the waves of a SIMD overlap the two anyway).
+// iteration later, the waves of a SIMD overlap the two anyway).  39 % MFMA and 42 % vector pipe busy, a third of the
+// waves' time is waits; four waves a SIMD (two key groups in one workgroup) spill: a wave holds 172 registers.
+// Few rows behind a long context leave most of the chip idle: there a tile's keys are shared by several workgroups
+// (FlashSplit; 100 rows behind 8000 keys 215 -> 41 us, 16 behind 2000 56 -> 16).
 #pragma once
 #include "common.h"
 
@@ -27,14 +30,21 @@ namespace la {
 constexpr int FL_KT = 64;  // keys per tile
 constexpr int FL_QT = 64;  // query rows per workgroup (the rows of a prefill work tile)
 
+// Keys split over grid.z: unnormalised sums [P][T][Hq][DH] and (maximum, sum) [P][T][Hq], merged by flash_merge_kernel.
+struct FlashSplit {
+  float* o;
+  float2* ml;
+  int T;
+};
+
 LA_DEV int flash_key(int m) { return (m & ~12) | ((m & 4) << 1) | ((m & 8) >> 1); }
 
-template <int DH, int HPW>
+template <int DH, int HPW, bool SPLIT>
 __global__ __launch_bounds__(HPW * 128) __attribute__((amdgpu_waves_per_eu(2))) void prefill_flash_kernel(
     const bf16* __restrict__ q, const bf16* __restrict__ kc, const bf16* __restrict__ vc,
     const int* __restrict__ tiles, const int* __restrict__ cu_q, const int* __restrict__ ctx_lens,
     const int* __restrict__ block_tables, int max_blocks, int Hq, int Hkv, int bs_shift, float sl2,
-    bf16* __restrict__ out) {
+    bf16* __restrict__ out, FlashSplit sp) {
   constexpr int NT = HPW * 128;
   constexpr int CH = DH / 8;                 // 16-byte chunks of a K row
   constexpr int KS = DH / 16;                // MFMA k steps of the score product
@@ -112,13 +122,16 @@ __global__ __launch_bounds__(HPW * 128) __attribute__((amdgpu_waves_per_eu(2))) 
     }
   };
 
-  pages(0);
-  load_tile(0);
-  pages(FL_KT);
-  store_tile(0, 0);
+  // this workgroup's keys: all, or an equal share of the tiles
+  const int share = SPLIT ? ((kend + FL_KT - 1) / FL_KT + (int)gridDim.z - 1) / (int)gridDim.z * FL_KT : 0;
+  const int kbeg = SPLIT ? (int)blockIdx.z * share : 0, klim = SPLIT ? min(kend, kbeg + share) : kend;
+  pages(kbeg);
+  load_tile(kbeg);
+  pages(kbeg + FL_KT);
+  store_tile(kbeg, 0);
   __syncthreads();
-  for (int k0 = 0, buf = 0; k0 < kend; k0 += FL_KT, buf ^= 1) {
-    if (k0 + FL_KT < kend) load_tile(k0 + FL_KT);
+  for (int k0 = kbeg, buf = 0; k0 < klim; k0 += FL_KT, buf ^= 1) {
+    if (k0 + FL_KT < klim) load_tile(k0 + FL_KT);
     pages(k0 + 2 * FL_KT);
     if (k0 <= qlast) {
       f32x16 sc[2];
@@ -180,12 +193,24 @@ __global__ __launch_bounds__(HPW * 128) __attribute__((amdgpu_waves_per_eu(2))) 
           o[nd] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, pf[kk], o[nd], 0, 0, 0);
         }
     }
-    if (k0 + FL_KT < kend) store_tile(k0 + FL_KT, buf ^ 1);
+    if (k0 + FL_KT < klim) store_tile(k0 + FL_KT, buf ^ 1);
     __syncthreads();
   }
 
   l += __shfl_xor(l, 32, 64);
   if (w0 + lq >= qlen) return;
+  if constexpr (SPLIT) {
+    const long at = ((long)blockIdx.z * sp.T + qbeg + row) * Hq + h;
+    if (lh == 0) sp.ml[at] = float2{m, l};
+    if (m == -INFINITY) return;               // none of its keys: nobody reads the sums
+#pragma unroll
+    for (int nd = 0; nd < ND; ++nd)
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        *(float4*)(sp.o + at * DH + 32 * nd + 8 * j + 4 * lh) =
+            float4{o[nd][4 * j], o[nd][4 * j + 1], o[nd][4 * j + 2], o[nd][4 * j + 3]};
+    return;
+  }
   const float inv = l > 0.f ? 1.f / l : 0.f;
   bf16* orow = out + ((long)(qbeg + row) * Hq + h) * DH;
 #pragma unroll
@@ -197,6 +222,47 @@ __global__ __launch_bounds__(HPW * 128) __attribute__((amdgpu_waves_per_eu(2))) 
       for (int i = 0; i < 4; ++i) v[i] = (bf16)(o[nd][4 * j + i] * inv);
       *(bf16x4*)(orow + 32 * nd + 8 * j + 4 * lh) = v;
     }
+}
+
+// out row = sum_p o_p exp2(m_p - m) / sum_p l_p exp2(m_p - m).  A workgroup per head and 256 / (DH / 4) rows of a work tile;
+// the loads of eight partials in flight (one after the other it took longer than the shares).
+template <int DH>
+__global__ __launch_bounds__(256) void flash_merge_kernel(FlashSplit sp, int P, const int* __restrict__ tiles,
+                                                          const int* __restrict__ cu_q, int Hq, bf16* __restrict__ out) {
+  constexpr int L4 = DH / 4, RP = 256 / L4;    // threads of a row, rows of a workgroup
+  const int s = tiles[2 * blockIdx.y], h = blockIdx.x;
+  const int r = tiles[2 * blockIdx.y + 1] + blockIdx.z * RP + threadIdx.x / L4;
+  const int qbeg = cu_q[s], qlen = cu_q[s + 1] - qbeg;
+  const int d = threadIdx.x % L4 * 4;
+  if (r >= qlen) return;
+  const long at = (long)(qbeg + r) * Hq + h, step = (long)sp.T * Hq;
+  float m = -INFINITY, l = 0.f;
+  float4 a = {0.f, 0.f, 0.f, 0.f};
+  for (int p0 = 0; p0 < P; p0 += 8) {
+    float2 v[8];
+    float4 x[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const long k = at + min(p0 + i, P - 1) * step;
+      v[i] = sp.ml[k];
+      x[i] = *(const float4*)(sp.o + k * DH + d);
+    }
+    float mn = m;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) mn = p0 + i < P ? fmaxf(mn, v[i].x) : mn;
+    const float w0 = m == -INFINITY ? 0.f : exp2f(m - mn);
+    l *= w0, a.x *= w0, a.y *= w0, a.z *= w0, a.w *= w0;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      if (p0 + i >= P || v[i].x == -INFINITY) continue;   // a share without keys wrote no sums
+      const float w = exp2f(v[i].x - mn);
+      l += v[i].y * w;
+      a.x += x[i].x * w, a.y += x[i].y * w, a.z += x[i].z * w, a.w += x[i].w * w;
+    }
+    m = mn;
+  }
+  const float inv = l > 0.f ? 1.f / l : 0.f;
+  *(bf16x4*)(out + at * DH + d) = bf16x4{(bf16)(a.x * inv), (bf16)(a.y * inv), (bf16)(a.z * inv), (bf16)(a.w * inv)};
 }
 
 }  // namespace la

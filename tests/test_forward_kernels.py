@@ -59,6 +59,16 @@ def test_prefill_flash(Hq, Hkv, Dh, BS, qlens, ctx):
         at += n
 
 
+@pytest.mark.parametrize("Hq,Hkv,Dh,BS", [(32, 8, 128, 32), (6, 6, 128, 16), (8, 2, 64, 128)])
+@pytest.mark.parametrize("qlens,ctx,shares", [([16], [2016], 7), ([5, 70], [1500, 130], 5), ([65, 1], [65, 4100], 15)])
+def test_prefill_shares(Hq, Hkv, Dh, BS, qlens, ctx, shares):
+    """The same behind long contexts, a tile's keys shared by several workgroups, some of them without keys (the short
+    sequences), with empty and with partly masked shares."""
+    blocks = max(-(-c // BS) for c in ctx)
+    assert ops._prefill_splits(sum(-(-n // 64) for n in qlens), Hq, Hkv, Dh, BS, blocks * BS, sum(qlens) // len(qlens)) >= min(shares, 8)
+    test_prefill_flash(Hq, Hkv, Dh, BS, qlens, ctx)
+
+
 def _weight(N, K, t, seed):
     w = np.random.default_rng(seed).standard_normal((N, K)).astype(np.float32) * 0.05
     return ops.QWeight.from_raw(quantize(w, t), t, (N, K), DEV, keep_ref=True)
