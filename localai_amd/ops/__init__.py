@@ -1372,11 +1372,13 @@ def glu_linear(x: torch.Tensor, ws: Sequence[QWeight], F: int, mode: int,
             return None
         out = torch.empty(M, F, dtype=torch.bfloat16, device=x.device)
         t_ref = _time_cold(lambda: act(linear_multi(x, ws), F, mode))
-        best, best_t = None, t_ref
+        # (fused, gate and up are not rounded before the activation: taken unless it is 5 % slower)
+        best, best_t = None, 1.05 * t_ref
         if w_ok([pair[0], pair[2]]) and pair[0].fmt == pair[2].fmt:
-            # the others lose at every size (28672 x 4096, Q4_K: 256 rows 73 us against 84 to 95, 128 rows 55 against 67 to
-            # 75), but one timed call now and then says otherwise
-            cands = [24, 22] if M > 128 else [22]
+            # 28672 x 4096, Q4_K, steps of 8 layers: 70 rows 107 1465 us, 22 1483, unfused 1462; 128 rows 1586, 1602, 1595;
+            # 250 rows 24 2357, 109 2346,
+            # unfused 2351 (alone, 256 rows: 24 73, 109 84 to 88)
+            cands = [24] if M > 128 else [107, 22] if q32_ok([pair[0]], 7) else [22]
         else:
             cands = [6, 7, 8] if M > 128 else [7, 12, 14]
         for t in cands:

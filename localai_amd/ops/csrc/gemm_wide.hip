@@ -23,8 +23,10 @@
 // are pinned behind the previous half-step; without that the compiler waits for every outstanding read: 78 -> 75 us),
 // the DMA's issue (one instruction after an MFMA, not all behind the barrier: -> 71 us), address arithmetic (scalar).
 // gate|up 28672 x 4096 of Q4_K with its activation: 256 rows 78 (gemm_bs.hip) -> 71 us, 128 rows 68 (gemm_q32.hip) ->
-// 52, 701 rows 229 (copy, library, activation) -> 200; 4096 x 14336 at 400 rows 115 (copy, library) -> 80, 4096 x 4096
-// 42 -> 36.  Plain products of up to 256 rows with few columns stay with the other kernels: the autotuner times them.
+// 55, 701 rows 229 (copy, library, activation) -> 208 with the first of these three steps and 6 % less with all; 4096 x
+// 14336 at 400 rows 115 (copy, library) -> 80, 4096 x 4096 42 -> 36.  Plain products of up to 256 rows with few columns
+// stay with the other kernels: the autotuner times them all.  Inside a step of 256 rows the gated product is level with
+// gemm_q32.hip's (2357 and 2346 us): there the weights' bytes in flight are the bound.
 #include <type_traits>
 
 #include "qstage.h"
