@@ -3823,12 +3823,11 @@ def moe_linear(x: torch.Tensor, mw: MoEWeights, order: torch.Tensor, off: torch.
 # MOE32_MIN_T tokens: gate|up with the SwiGLU fused (bf16 h in grouped row order), then the
 # routing-weighted down projection.  Variant ids: gemm_q32.hip moe32_var.
 MOE32 = os.environ.get("LOCALAI_AMD_MOE32", "1") == "1"
-# Variant by batch (scripts/moe_bench.py, Mixtral-8x7B shapes, gpurun_out/r5_moe32_bench.log):
+# Variant by batch (scripts/moe_bench.py, Mixtral-8x7B shapes):
 # T = 64: 32-row tiles, 4 workgroups per CU (var 9) 156 + 86 us vs the 16-column kernel's
 # 285 + 9 (act) + 143; T = 128 / 256: 64-row tiles in 8-wave workgroups (var 4) 180 + 91 /
 # 291 + 162 us vs 276 + 15 + 145 / 470 + 16 + 255.
 # T = 16 / 24 / 32: var 9 232 / 234 / 237 us vs 266 / 315 / 317; T = 8: 221 vs 212
-# (gpurun_out/r5_moe_small.log)
 MOE32_MIN_T = int(os.environ.get("LOCALAI_AMD_MOE32_MIN_T", "12"))
 MOE32_SMALL_T = 48     # below: var 9 (32-row tiles); from here: var 17 (64-row chunks, live row blocks)
 MOE32_LIVE_BIG_T = 192  # from here: var 19 (one 128-row chunk per expert at top-2 of 8)

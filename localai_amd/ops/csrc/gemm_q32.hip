@@ -997,7 +997,7 @@ static int moe32_launch(int var, const QW* qws, int N, int K, int E, const int* 
                         const bf16* X, int ldx, int maxM, int splits, const float* wts, float* out, bf16* outb,
                         int ldo, long slab, int act, hipStream_t st) {
   const int KS = K >> 6, per = (KS + splits - 1) / splits;
-  // 64 columns per wave at 128 rows spill with Q6_K / Q8_0's larger fragment state: those formats
+  // 64 columns per wave in 4 waves at 128 rows spill with the larger fragments of Q6_K / Q8_0: those formats
   // take the 32-column form of the same chunking
   if (FMT != FMT_Q4_K && var == 20) var -= 4;
   return moe32_var<FMT == FMT_Q4_K>(var, [&](auto c) {
